@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define KITTY_ABI_VERSION 6
+#define KITTY_ABI_VERSION 7
 
 /* Element type of 16-bit data (the *_dtype fields below). */
 #define KITTY_DTYPE_F16 0
@@ -329,6 +329,31 @@ typedef struct {
 } kitty_append_args;
 
 int kitty_append_tokens(const kitty_append_args *args, kitty_stream_t stream);
+
+/* ------------------------------------------------- prompt attention
+ * Replaces the scaled_dot_product_attention call of the T > 1 branch of
+ * KittyPagedAttention.forward (kitty/attention.py:179-191; ABI version 7):
+ * out[b, h, i] = softmax over j <= i of (q[b, h, i] . k[b, kh, j] * sm_scale)
+ * times v[b, kh, j], kh = h / (num_q_heads / num_kv_heads), with fp32 scores,
+ * softmax and sums, converted to the inputs' type.  head_dim 128; q, k and v
+ * 16-byte aligned with strides that are multiples of 8 elements, out 8-byte
+ * aligned with strides that are multiples of 4; token strides of k and v
+ * non-negative with a head's rows inside 2 GiB; other layouts return
+ * KITTY_E_UNSUPPORTED.  Scores that are NaN or +infinity give NaN rows, as
+ * the softmax does; a NaN or infinite value row j may also reach rows
+ * i < j of the same 64-token tile (their weight 0 times it), and an infinite
+ * value gives NaN where the plain product would give infinity. */
+typedef struct {
+    const uint16_t *q, *k, *v; /* (B, Hq, T, D), (B, Hkv, T, D) twice */
+    uint16_t *out;             /* (B, Hq, T, D) */
+    int64_t q_s_seq, q_s_head, q_s_tok, k_s_seq, k_s_head, k_s_tok, v_s_seq, v_s_head, v_s_tok;
+    int64_t o_s_seq, o_s_head, o_s_tok;
+    int32_t batch, num_q_heads, num_kv_heads, tokens, head_dim;
+    int32_t dtype; /* KITTY_DTYPE_F16 or KITTY_DTYPE_BF16: q, k, v and out */
+    float sm_scale;
+} kitty_prefill_args;
+
+int kitty_prefill_attention(const kitty_prefill_args *args, kitty_stream_t stream);
 
 /* ------------------------------------------------ spill bookkeeping
  * The device side of the page-table and counter updates that

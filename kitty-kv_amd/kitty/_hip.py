@@ -19,7 +19,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # KITTY_HIP_LIBRARY selects another build of the same ABI (e.g. a tuning variant).
 LIB_PATH = os.environ.get("KITTY_HIP_LIBRARY") or os.path.join(_HERE, "libkitty_hip.so")
 
-KITTY_ABI_VERSION = 6
+KITTY_ABI_VERSION = 7
 KITTY_OK = 0
 KITTY_E_INVALID = -1
 KITTY_E_HIP = -2
@@ -118,13 +118,26 @@ class AppendArgs(ctypes.Structure):
     ]
 
 
+class PrefillArgs(ctypes.Structure):
+    """kitty_prefill_args: causal attention of a prompt."""
+    _fields_ = [
+        ("q", _vp), ("k", _vp), ("v", _vp), ("out", _vp),
+        ("q_s_seq", _i64), ("q_s_head", _i64), ("q_s_tok", _i64),
+        ("k_s_seq", _i64), ("k_s_head", _i64), ("k_s_tok", _i64),
+        ("v_s_seq", _i64), ("v_s_head", _i64), ("v_s_tok", _i64),
+        ("o_s_seq", _i64), ("o_s_head", _i64), ("o_s_tok", _i64),
+        ("batch", _i32), ("num_q_heads", _i32), ("num_kv_heads", _i32), ("tokens", _i32), ("head_dim", _i32),
+        ("dtype", _i32), ("sm_scale", ctypes.c_float),
+    ]
+
+
 EXPORTED_SYMBOLS = (
     "kitty_abi_version", "kitty_last_error", "kitty_quantize_kv_blocks",
     "kitty_dequantize_key_page", "kitty_dequantize_value_page",
     "kitty_decode_workspace_size", "kitty_decode_path", "kitty_paged_decode", "kitty_paged_decode_splits",
     "kitty_paged_decode_merge", "kitty_paged_decode_noalloc", "kitty_append_tokens", "kitty_channel_abs_sum",
     "kitty_channel_abs_sum_workspace_size", "kitty_channel_abs_sum_deferred_size", "kitty_channel_abs_sum_deferred",
-    "kitty_channel_abs_sum_flush", "kitty_store_i32",
+    "kitty_channel_abs_sum_flush", "kitty_store_i32", "kitty_prefill_attention",
 )
 
 _lib: Optional[ctypes.CDLL] = None
@@ -163,6 +176,7 @@ def load() -> ctypes.CDLL:
     L.kitty_channel_abs_sum_deferred.argtypes = L.kitty_channel_abs_sum.argtypes
     L.kitty_channel_abs_sum_flush.argtypes = [_vp, _i32, _i32, _vp, _vp]
     L.kitty_store_i32.argtypes = [_vp, _vp, _i32, _vp]
+    L.kitty_prefill_attention.argtypes = [ctypes.POINTER(PrefillArgs), _vp]
     if L.kitty_abi_version() != KITTY_ABI_VERSION:
         raise ImportError(f"libkitty_hip ABI {L.kitty_abi_version()} != {KITTY_ABI_VERSION}")
     _lib = L

@@ -19,8 +19,10 @@ Prefill (T > 1): the chunk goes into the pipeline in bulk (sinks and buffer
 rows copied, every complete page quantised straight from the chunk in one
 launch per sequence; the same state as pushing the tokens one at a time,
 which is what the reference does, ``:169-177``), and the output is causal
-attention over the chunk, as the reference computes it (``:179-191``); it
-runs in float32 (torch's SDPA math path).
+attention over the chunk, as the reference computes it (``:179-191``), with
+scores, softmax and sums in float32: fp16 and bf16 prompts at head_dim 128
+run ``kitty_prefill_attention``, everything else (other head_dims, float32,
+inputs that need gradients) torch's scaled_dot_product_attention.
 
 Pools and buffers on the CPU (``KittyConfig.device = "cpu"``, the reference's
 config-1 plumbing case) run the same steps with the torch code of
@@ -38,7 +40,7 @@ import torch.nn.functional as F
 from .config import KittyConfig
 from .layout import PageCentricKVLayoutManager
 from .pipeline import KittyInferencePipeline
-from .kernels.ops import DecodePlan, boost_rows_unique, decode_plan
+from .kernels.ops import DecodePlan, boost_rows_unique, decode_plan, prefill_attention, prefill_supported
 
 
 class KittyPagedAttention(nn.Module):
@@ -102,6 +104,8 @@ class KittyPagedAttention(nn.Module):
 
     def _prefill(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, seq_ids: List[int]) -> torch.Tensor:
         self.pipeline.push_chunk(self.layer_id, k, v, seq_ids)
+        if prefill_supported(q, k, v):
+            return prefill_attention(q, k, v, self.scale)
         k_exp = k.float().repeat_interleave(self.q_per_kv, dim=1)
         v_exp = v.float().repeat_interleave(self.q_per_kv, dim=1)
         out = F.scaled_dot_product_attention(q.float(), k_exp, v_exp, attn_mask=None, dropout_p=0.0,

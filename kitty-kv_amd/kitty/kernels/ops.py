@@ -17,6 +17,7 @@ from typing import Optional, Sequence, Tuple
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from .. import _hip
 from . import cpu
@@ -431,6 +432,47 @@ def decode_plan(*args, **kwargs):
 def paged_decode(*args, **kwargs) -> torch.Tensor:
     """Batched fused paged decode attention: ``decode_plan(*args, **kwargs).run()``."""
     return decode_plan(*args, **kwargs).run()
+
+
+def prefill_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """True when kitty_prefill_attention takes these (B, heads, T, D) tensors
+    as they are: head_dim 128, one 16-bit dtype, 16-byte rows.  Anything a
+    plain kernel launch would drop stays with torch: inputs that need
+    gradients, forward-mode tangents, functorch transforms, tensor subclasses
+    (fake tensors) and negated or conjugated views."""
+    if not (type(q) is type(k) is type(v) is torch.Tensor and q.device.type == "cuda" and q.device == k.device == v.device):
+        return False
+    if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype:
+        return False
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+        return False
+    if forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    if not (q.dim() == k.dim() == v.dim() == 4 and q.shape[3] == k.shape[3] == 128 and k.shape == v.shape
+            and q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2] and q.shape[2] > 0
+            and q.shape[1] > 0 and k.shape[1] > 0 and q.shape[1] % k.shape[1] == 0):
+        return False
+    for t in (q, k, v):
+        # a stride of a dimension of size 1 is never used for an address past the row
+        if t.is_neg() or t.stride(3) != 1 or t.data_ptr() % 16 or any(s % 8 for s in t.stride()[:3]):
+            return False
+    # 32-bit byte offsets inside a head (kitty_prefill_attention); the launch's grid
+    T = q.shape[2]
+    return all(0 <= s and (T + 64) * s * 2 + 256 < 1 << 31 for s in (k.stride(2), v.stride(2))) \
+        and q.shape[0] * q.shape[1] * (T + 127) < 1 << 31
+
+
+def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sm_scale: float) -> torch.Tensor:
+    """Causal attention of a prompt, (B, Hq, T, D) like q
+    (kitty_prefill_attention; the caller checked prefill_supported)."""
+    B, Hq, T, D = q.shape
+    out = torch.empty(B, Hq, T, D, dtype=q.dtype, device=q.device)
+    if B == 0:
+        return out
+    a = _hip.PrefillArgs(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), *q.stride()[:3], *k.stride()[:3],
+                         *v.stride()[:3], *out.stride()[:3], B, Hq, k.shape[1], T, D, _hip.dtype_code(q, "q"), sm_scale)
+    _hip.check(_hip.load().kitty_prefill_attention(ctypes.byref(a), _hip.stream_ptr(q.device)))
+    return out
 
 
 def decode_workspace_bytes(B: int, Hq: int, Hkv: int, D: int, G: int, Dk: int, max_pages: int,
