@@ -183,7 +183,8 @@ int kitty_dequantize_value_page(const kitty_page_store *store, int64_t page, int
  * as fp16 (two rows: product and exact residual), and 2^-1 q[d] * s_k[d] for
  * a boosted channel's high bits, so |q[d] * s_k[d]| must stay below 2^17
  * (131,072) on boosted channels and 2^19 on the others; beyond that the
- * scores of that head are not finite.  The generic kernel computes in fp32.
+ * scores of that head are not finite.  bf16 operands are scaled by powers of
+ * two first and have no such range; the generic kernel computes in fp32.
  *
  * Pools must be the contiguous tensors of PageCentricKVLayoutManager (16-byte
  * aligned bases); page ids are int32 and byte offsets are 64-bit, so a pool
@@ -247,7 +248,7 @@ typedef struct {
 
     /* element types (ABI version 3): the metadata pools, and q with the
      * sinks and tails.  out is fp16 either way, as the reference returns
-     * (kitty/kernels/attention.py:189).  bf16 runs the shape-generic kernel. */
+     * (kitty/kernels/attention.py:189). */
     int32_t meta_dtype; /* KITTY_DTYPE_F16 or KITTY_DTYPE_BF16 */
     int32_t act_dtype;  /* KITTY_DTYPE_F16 or KITTY_DTYPE_BF16 */
 } kitty_decode_args;
@@ -261,8 +262,11 @@ int kitty_paged_decode(const kitty_decode_args *args, kitty_stream_t stream);
  * sub-groups of 16 heads, one pass over the pages each, through
  * kitty_paged_decode only), fp16,
  * 16-byte aligned buffers, unique boost
- * ranks) or KITTY_DECODE_PATH_GENERIC (every other shape the reference
- * accepts, about 15x slower at the production shape).  Mirrors the
+ * ranks) or KITTY_DECODE_PATH_GENERIC (everything else: the shape-generic
+ * kernel, about 15x slower at the production shape, and, where only the
+ * element type keeps a call from the production kernel (q, sinks, tails and
+ * metadata all bf16), its bf16 instance, which carries probabilities and
+ * scores with the generic kernel's fp32 accuracy).  Mirrors the
  * dispatch decision of paged_attention (kitty/kernels/attention.py:320-341),
  * so callers can see when a profile with repeated ranks or a misaligned
  * buffer sends decode to the slower kernel. */

@@ -254,18 +254,39 @@ extern "C" int kitty_decode_path(const kitty_decode_args *args, int32_t *path)
         return rc;
     if (!path)
         return fail(KITTY_E_INVALID, "path is NULL");
-    *path = mfma_path_supported(p) ? KITTY_DECODE_PATH_MFMA : KITTY_DECODE_PATH_GENERIC;
+    // bf16 buffers run a bf16 instance of the MFMA split kernel, but report GENERIC (kitty_hip.h)
+    *path = mfma_path_supported(p) && !p.act_bf16 ? KITTY_DECODE_PATH_MFMA : KITTY_DECODE_PATH_GENERIC;
     return KITTY_OK;
 }
 
-static int prepare(const kitty_decode_args *args, DecodeParams &p)
+// Parameters of a call that has `bytes` of workspace, and what it needs.  The
+// bf16 instance of the MFMA kernel needs more than the generic kernel for
+// many short sequences; a workspace that only the generic kernel's partials fit
+// runs that kernel (which is what bf16 ran before the instance existed).
+static int build_fitting(const kitty_decode_args *args, DecodeParams &p, size_t bytes, size_t &need)
 {
     int rc = build_params(args, p);
     if (rc || p.B == 0)
         return rc;
+    need = workspace_need(p, *args, false);
+    if (need > bytes && p.act_bf16 && mfma_path_supported(p)) {
+        kitty_decode_args generic = *args;
+        generic.flags &= ~KITTY_DECODE_UNIQUE_BOOST_ROWS;
+        rc = build_params(&generic, p);
+        if (rc == KITTY_OK)
+            need = workspace_need(p, generic, false);
+    }
+    return rc;
+}
+
+static int prepare(const kitty_decode_args *args, DecodeParams &p)
+{
+    size_t need = 0;
+    int rc = build_fitting(args, p, args ? args->workspace_bytes : 0, need);
+    if (rc || p.B == 0)
+        return rc;
     if (!args->q || !args->out || !args->num_pages || !args->boost_idx || !args->sink_len || !args->tail_len)
         return fail(KITTY_E_INVALID, "NULL q, out, num_pages, boost_idx, sink_len or tail_len");
-    const size_t need = workspace_need(p, *args, false);
     if (!args->workspace || args->workspace_bytes < need)
         return fail(KITTY_E_INVALID, "workspace too small: need " + std::to_string(need) + " bytes");
     if ((uintptr_t)args->workspace & 15)
@@ -355,10 +376,10 @@ static int scratch_address(void **out)
 extern "C" int kitty_paged_decode_noalloc(const kitty_decode_args *args, kitty_stream_t stream)
 {
     DecodeParams p;
-    int rc = build_params(args, p);
+    size_t need = 0;
+    int rc = build_fitting(args, p, kScratchBytes, need);
     if (rc || p.B == 0)
         return rc;
-    const size_t need = workspace_need(p, *args, false);
     if (need > kScratchBytes)
         return fail(KITTY_E_INVALID, "kitty_paged_decode_noalloc: this batch needs " + std::to_string(need) +
                                          " bytes of scratch, the maximum is " + std::to_string(kScratchBytes) +

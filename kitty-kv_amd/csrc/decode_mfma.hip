@@ -34,6 +34,12 @@
 //       those units at each page, and 2^24 4^-a is applied when the
 //       segment's partial is written.
 //
+// bf16 (q, sinks, tails and metadata all bf16): an instance of the same kernel
+// that keeps the fp32 accuracy of the generic kernel it replaces at this
+// shape (page_qk, qk_setup, pv_split say how).  8 sequences of 3,000-9,000
+// tokens, 32 query / 8 KV heads: 27.9 us split (generic kernel: 119.6), the whole
+// decode 28.7 us against 115.9, both 2.1e-4 off float64 (the output rounding).
+//
 // Reduction index k of every MFMA follows the natural channel / token order
 // within a 32-wide step (the tr8 row order puts even and odd bytes of a
 // word on consecutive k).
@@ -51,6 +57,7 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef short s16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // LDS stage of one (page, head) record, byte offsets.
 constexpr int kKlo = 0;       // key low bits   (128 rows x 32 B), chunk-swizzled
@@ -114,6 +121,45 @@ __device__ __forceinline__ half8 slot_codes(const RawCodes &r, int a)
                                                                                   : codes_to_half8<3>(r);
 }
 
+// The bf16 instances' codes: slots 0 and 1 moved up to the places of slots 2
+// and 3 (code 4^(2 + a % 2) 2^-24), two shifts more per word.  The matrix core
+// aligns a block's products by the exponents of their operands before it
+// adds, and a subnormal counts with the smallest normal exponent: a code of
+// slot 0 sits ten bits below that, and its sums keep 14 bits where slot 3's
+// keep 20 (measured score errors: 1e-4, 2.5e-5, 5e-6 and 1e-6 for slots 0 to 3).
+constexpr int bf_slot(int a) { return 2 + (a & 1); }
+
+struct RawCodesUp {
+    RawCodes r, up;
+};
+
+__device__ __forceinline__ RawCodesUp raw_codes_up(i32x2 raw)
+{
+    const unsigned w0 = (unsigned)raw[0], w1 = (unsigned)raw[1];
+    return RawCodesUp{raw_codes(raw), RawCodes{{w0 << 4, w1 << 4, w0 >> 4, w1 >> 4}}};
+}
+
+__device__ __forceinline__ half8 slot_codes(const RawCodesUp &r, int a)
+{
+    return a == 0 ? codes_to_half8<2>(r.up) : a == 1 ? codes_to_half8<3>(r.up) : a == 2 ? codes_to_half8<2>(r.r)
+                                                                                          : codes_to_half8<3>(r.r);
+}
+
+// Codes of the production (fp16) and the bf16 instances, and 4^slot of their scale.
+template <bool BF>
+__device__ __forceinline__ auto page_codes(i32x2 raw)
+{
+    if constexpr (BF)
+        return raw_codes_up(raw);
+    else
+        return raw_codes(raw);
+}
+template <bool BF>
+__device__ __forceinline__ constexpr float slot_weight(int a)
+{
+    return (float)(1 << (2 * (BF ? bf_slot(a) : a)));
+}
+
 // PV operands of the GQA-4 path (v_mfma_f32_16x16x128_f8f6f4, A fp8 e4m3,
 // B fp4 e2m1).  A 2-bit value code in the low bits of a nibble whose top
 // two bits are clear is the e2m1 number code / 2, so value codes become B
@@ -155,6 +201,21 @@ __device__ __forceinline__ void fp8_residual(float *x, unsigned w, float scale)
 __device__ __forceinline__ f32x4 mfma(half8 a, half8 b, f32x4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ f32x4 mfma_bf(bf16x8 a, bf16x8 b, f32x4 c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// The two halves of a word of bf16 values as fp32 (exact).
+__device__ __forceinline__ float bf_lo(unsigned w) { return __builtin_bit_cast(float, w << 16); }
+__device__ __forceinline__ float bf_hi(unsigned w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
+
+// Two fp32 values as packed fp16, rounded toward zero.
+__device__ __forceinline__ unsigned pack_rtz(float a, float b)
+{
+    return __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(a, b));
 }
 
 template <int CTRL>
@@ -272,16 +333,17 @@ __device__ __forceinline__ void wait_vmcnt()
 }
 
 // Running state of one wave across its pages.
-template <int GQ>
+template <int GQ, bool BF>
 struct WaveState {
     static constexpr int HPL = GQ / 4;      // heads per lane group
     u32x4 qv[4], qvh;                        // static halves of the QK A operand (fp16 q)
-    float qk_c;                              // sm_scale * log2(e): scores in log2 units
+    float qk_c[BF ? HPL : 1];                // sm_scale * log2(e): scores in log2 units (bf16: times the head's 2^E)
     int hch[8];                              // channel of high-bit row 8q + i
     int tr_base0, tr_base1;                  // tr8 source offsets (byte columns 0-15 / 16-31)
     int prow;                                // head row whose P' this lane reads for PV
     float m_run[HPL], l_run[HPL];
     f32x4 O[2][4];                           // GQA 8 / 16: output tiles (4^a O of channels 64cb + 4r + a)
+    float ob[2][4][HPL];                     // bf16: O of head slot j, channels 64cb + 4r + a
     float o4[4][2];                          // GQA 4: O of head q, channels 32ch + 2r + e
     int trv[2][2];                           // GQA 4: tr4 offsets of value rows 32q + 16k + r, 16-byte chunk c
 };
@@ -300,7 +362,7 @@ struct WaveState {
 //  O[h][d] += 2 sig (C0 + C1 / 16 + C2 / 256) - sum_t P'_t z_t, C_t = row
 //  4h + t of the MFMA output (fp4 value = code / 2).
 template <int GQ>
-__device__ __forceinline__ void pv_fp8_fp4(WaveState<GQ> &W, unsigned char *st, const f32x4 (&S)[2][4],
+__device__ __forceinline__ void pv_fp8_fp4(WaveState<GQ, false> &W, unsigned char *st, const f32x4 (&S)[2][4],
                                            const f32x4 &Yt, int lane)
 {
     const int q = lane >> 4, r = lane & 15;
@@ -320,14 +382,14 @@ __device__ __forceinline__ void pv_fp8_fp4(WaveState<GQ> &W, unsigned char *st, 
     for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
         for (int a = 0; a < 4; ++a)
-            sv[cb][a] = (S[cb][a][0] + S[cb][a][1]) * (W.qk_c * (kSub / (float)(1 << (2 * a))));
+            sv[cb][a] = (S[cb][a][0] + S[cb][a][1]) * (W.qk_c[0] * (kSub / (float)(1 << (2 * a))));
     float mx = sv[0][0];
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
         for (int a = 0; a < 4; ++a)
             mx = fmaxf(mx, sv[cb][a]);
-    const float yk = (Yt[0] + Yt[1]) * W.qk_c;
+    const float yk = (Yt[0] + Yt[1]) * W.qk_c[0];
     mx = row_max16(mx) - yk;
     const float mn = fmaxf(W.m_run[0], mx);
     const float alpha = __builtin_amdgcn_exp2f(W.m_run[0] - mn);
@@ -408,10 +470,48 @@ __device__ __forceinline__ void pv_fp8_fp4(WaveState<GQ> &W, unsigned char *st, 
 // sum_k A c for tokens 64 cb + 4 r + a on the head rows (rounded product and
 // residual rows, or one row and a second chain at GQA 16), Yt the
 // zero-point term Y per head row.
-template <int GQ>
-__device__ __forceinline__ void page_qk(const WaveState<GQ> &W, const unsigned char *st, int lane, int Dk,
-                                        f32x4 (&S)[2][4], f32x4 &Yt)
+//
+// bf16 metadata: the page's 128 scales and 128 zero points are converted to
+// fp16 in the stage first, two of each pair of channels per lane (converted
+// where they are read, each of the 16 lanes of a group would redo its
+// 40 words: 120 VALU against 12).  q enters times 2^9 (qk_setup), so that the
+// products and their residuals stay clear of fp16's subnormals.  A page
+// with a scale of 16 or more is brought below it by a power of two, 1 / kmul,
+// which the scores take back, so any bf16 scale decodes.
+template <int GQ, bool BF>
+__device__ __forceinline__ void page_qk(const WaveState<GQ, BF> &W, unsigned char *st, int lane, int Dk,
+                                        f32x4 (&S)[2][4], f32x4 &Yt, float &kmul)
 {
+    kmul = 1.0f;
+    if constexpr (BF) {
+        // lanes 0-31: scales of channels 4 lane .. + 3, lanes 32-63: zero
+        // points (inline asm: see compute_page)
+        unsigned w0, w1;
+        {
+            uint64_t w;
+            const unsigned addr = (unsigned)(uintptr_t)(st + kMeta + 8 * lane);
+            asm volatile("ds_read_b64 %0, %1\n\t"
+                         "s_waitcnt lgkmcnt(0)"
+                         : "=v"(w)
+                         : "v"(addr)
+                         : "memory");
+            w0 = (unsigned)w, w1 = (unsigned)(w >> 32);
+        }
+        const unsigned mag = max(max(w0 << 16 & 0x7fffffffu, w0 & 0x7fff0000u), max(w1 << 16 & 0x7fffffffu, w1 & 0x7fff0000u));
+        float f0 = bf_lo(w0), f1 = bf_hi(w0), f2 = bf_lo(w1), f3 = bf_hi(w1);
+        if (__builtin_expect(__ballot(lane < 32 && mag >= 0x41800000u) != 0, 0)) {
+            int e = lane < 32 ? (int)(mag >> 23) : 0;   // biased exponent
+            for (int off = 1; off < 64; off <<= 1)
+                e = max(e, __shfl_xor(e, off));
+            const int k = e - 130;                      // the largest scale below 2^4
+            kmul = __builtin_amdgcn_ldexpf(1.0f, k);
+            if (lane < 32) {
+                f0 = __builtin_amdgcn_ldexpf(f0, -k), f1 = __builtin_amdgcn_ldexpf(f1, -k);
+                f2 = __builtin_amdgcn_ldexpf(f2, -k), f3 = __builtin_amdgcn_ldexpf(f3, -k);
+            }
+        }
+        *(uint2 *)(st + kMeta + 8 * lane) = make_uint2(pack_rtz(f0, f1), pack_rtz(f2, f3));
+    }
     const int q = lane >> 4;
 
     // ---------------- operands from LDS, issued together
@@ -493,7 +593,7 @@ __device__ __forceinline__ void page_qk(const WaveState<GQ> &W, const unsigned c
     for (int s = 0; s < 4; ++s)
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) {
-            const RawCodes rc = raw_codes(kraw[s][cb]);
+            const auto rc = page_codes<BF>(kraw[s][cb]);
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
                 const half8 kc = slot_codes(rc, a);
@@ -505,7 +605,7 @@ __device__ __forceinline__ void page_qk(const WaveState<GQ> &W, const unsigned c
     if (Dk > 0) {
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb) {
-            const RawCodes rc = raw_codes(hraw[cb]);
+            const auto rc = page_codes<BF>(hraw[cb]);
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
                 const half8 kc = slot_codes(rc, a);
@@ -519,15 +619,153 @@ __device__ __forceinline__ void page_qk(const WaveState<GQ> &W, const unsigned c
     __builtin_amdgcn_s_setprio(0);
 }
 
+// bf16: online softmax and PV of one page with fp16 MFMAs and P'
+// = p * s_t in two fp16 terms (value rounded toward zero, and its remainder:
+// 21 bits, nothing lost against the fp32 probabilities of the generic
+// kernel).  P' enters scaled by 2^(15 - e), s_max < 2^e the page's largest value scale, so
+// it stays below 2^15 whatever range bf16 scales have.  GQA 4 and 8 put the
+// terms on the first two MFMA rows of each head, GQA 16 runs a second chain; a
+// page's output tiles start at zero and are folded into O in fp32.  (GQA 4 on
+// the fp8 x fp4 MFMAs of the fp16 instance, with a fourth term, kept errors of
+// 4-6e-4 where the generic kernel has 2e-4: those sums hold too few bits.)
 template <int GQ>
-__device__ __forceinline__ void compute_page(WaveState<GQ> &W, unsigned char *st, int lane, int Dk)
+__device__ __forceinline__ void pv_split(WaveState<GQ, true> &W, unsigned char *st, const f32x4 (&S)[2][4],
+                                         const f32x4 &Yt, float kmul, int lane)
+{
+    constexpr int HPL = GQ / 4;
+    constexpr int RSTEP = 4 / HPL;
+    const int q = lane >> 4, r = lane & 15;
+    i32x2 vraw[4][2];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        vraw[s][0] = tr8(st + kVal + 1024 * s + W.tr_base0);
+        vraw[s][1] = tr8(st + kVal + 1024 * s + W.tr_base1);
+    }
+    const u32x4 vm0 = *(const u32x4 *)(st + kMeta + 512 + 4 * (4 * r));
+    const u32x4 vm1 = *(const u32x4 *)(st + kMeta + 512 + 4 * (64 + 4 * r));
+    float smax = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+        smax = fmaxf(smax, fmaxf(bf_lo(vm0[a]), bf_lo(vm1[a])));
+    const int e15 = __builtin_amdgcn_frexp_expf(row_max16(smax)) - 15;
+    const float down = __builtin_amdgcn_ldexpf(1.0f, -e15);
+    float alpha[HPL], yv[HPL];
+#pragma unroll
+    for (int j = 0; j < HPL; ++j) {
+        const int ri = j * RSTEP;
+        const float qk_c = W.qk_c[j] * kmul;
+        float sv[2][4];
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                sv[cb][a] = (GQ == 16 ? S[cb][a][ri] : S[cb][a][ri] + S[cb][a][ri + 1]) *
+                            (qk_c * (kSub / slot_weight<true>(a)));
+        float mx = sv[0][0];
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                mx = fmaxf(mx, sv[cb][a]);
+        const float yk = (GQ == 16 ? Yt[ri] : Yt[ri] + Yt[ri + 1]) * qk_c;
+        mx = row_max16(mx) - yk;
+        const float mn = fmaxf(W.m_run[j], mx);
+        alpha[j] = __builtin_amdgcn_exp2f(W.m_run[j] - mn);
+        W.m_run[j] = mn;
+        const float mny = mn + yk;
+        float lsum = 0.0f, ysum = 0.0f;
+        const int h = q * HPL + j;
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb) {
+            const u32x4 vm = cb ? vm1 : vm0;
+            float x[4];
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const float pr = __builtin_amdgcn_exp2f(sv[cb][a] - mny);
+                lsum += pr;
+                x[a] = pr * bf_lo(vm[a]);
+                ysum = __builtin_fmaf(x[a], bf_hi(vm[a]), ysum);
+                x[a] *= down;
+            }
+            const unsigned h0 = pack_rtz(x[0], x[1]), h1 = pack_rtz(x[2], x[3]);
+            const unsigned l0 = pack_rtz(x[0] - (float)as_h2(h0)[0], x[1] - (float)as_h2(h0)[1]);
+            const unsigned l1 = pack_rtz(x[2] - (float)as_h2(h1)[0], x[3] - (float)as_h2(h1)[1]);
+            // rows over the consumed key codes (GQA 16: the second terms over the value codes, read above)
+            unsigned char *hi = st + kKlo + 256 * (16 / GQ * h) + 2 * (64 * cb + 4 * r);
+            *(uint2 *)hi = make_uint2(h0, h1);
+            *(uint2 *)(GQ == 16 ? hi + (kVal - kKlo) : hi + 256) = make_uint2(l0, l1);
+        }
+        W.l_run[j] = W.l_run[j] * alpha[j] + lsum;
+        yv[j] = row_sum16(ysum);
+    }
+    // A operand: row r of the terms (inline asm for the reason given in compute_page)
+    __builtin_amdgcn_s_setprio(1);
+    half8 Ap[4], Al[GQ == 16 ? 4 : 1];
+    {
+        const unsigned addr = (unsigned)(uintptr_t)(st + kKlo + 256 * r + 16 * q);
+        asm volatile("ds_read_b128 %0, %4\n\t"
+                     "ds_read_b128 %1, %4 offset:64\n\t"
+                     "ds_read_b128 %2, %4 offset:128\n\t"
+                     "ds_read_b128 %3, %4 offset:192\n\t"
+                     "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(Ap[0]), "=&v"(Ap[1]), "=&v"(Ap[2]), "=&v"(Ap[3])
+                     : "v"(addr)
+                     : "memory");
+        if constexpr (GQ == 16) {
+            const unsigned addr_l = addr + (kVal - kKlo);
+            asm volatile("ds_read_b128 %0, %4\n\t"
+                         "ds_read_b128 %1, %4 offset:64\n\t"
+                         "ds_read_b128 %2, %4 offset:128\n\t"
+                         "ds_read_b128 %3, %4 offset:192\n\t"
+                         "s_waitcnt lgkmcnt(0)"
+                         : "=&v"(Al[0]), "=&v"(Al[1]), "=&v"(Al[2]), "=&v"(Al[3])
+                         : "v"(addr_l)
+                         : "memory");
+        }
+    }
+    const float up = __builtin_amdgcn_ldexpf(kSub, e15);  // tile a holds slot_weight(a) 2^-24 2^-e15 sum P' c
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+        f32x4 T[4];
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+            T[a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const auto rc = page_codes<true>(vraw[s][cb]);
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const half8 vc = slot_codes(rc, a);
+                T[a] = mfma(Ap[s], vc, T[a]);
+                if constexpr (GQ == 16)
+                    T[a] = mfma(Al[s], vc, T[a]);
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int j = 0; j < HPL; ++j) {
+                const float t = GQ == 16 ? T[a][j * RSTEP] : T[a][j * RSTEP] + T[a][j * RSTEP + 1];
+                W.ob[cb][a][j] = __builtin_fmaf(W.ob[cb][a][j], alpha[j],
+                                                __builtin_fmaf(t, up * (1.0f / slot_weight<true>(a)), -yv[j]));
+            }
+    }
+    __builtin_amdgcn_s_setprio(0);
+}
+
+template <int GQ, bool BF>
+__device__ __forceinline__ void compute_page(WaveState<GQ, BF> &W, unsigned char *st, int lane, int Dk)
 {
     constexpr int HPL = GQ / 4;
     constexpr int RSTEP = 4 / HPL;  // accumulator register of head slot j = j * RSTEP
     const int q = lane >> 4, r = lane & 15;
     f32x4 S[2][4], Yt;
-    page_qk<GQ>(W, st, lane, Dk, S, Yt);
-    if constexpr (GQ == 4) {
+    float kmul;
+    page_qk<GQ, BF>(W, st, lane, Dk, S, Yt, kmul);
+    if constexpr (BF) {
+        pv_split<GQ>(W, st, S, Yt, kmul, lane);
+        return;
+    } else if constexpr (GQ == 4) {
         pv_fp8_fp4(W, st, S, Yt, lane);
         return;
     }
@@ -556,7 +794,7 @@ __device__ __forceinline__ void compute_page(WaveState<GQ> &W, unsigned char *st
 #pragma unroll
             for (int a = 0; a < 4; ++a)
                 sv[cb][a] = (GQ == 16 ? S[cb][a][ri] : S[cb][a][ri] + S[cb][a][ri + 1]) *
-                            (W.qk_c * (kSub / (float)(1 << (2 * a))));
+                            (W.qk_c[0] * (kSub / (float)(1 << (2 * a))));
         float mx = sv[0][0];
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb)
@@ -564,7 +802,7 @@ __device__ __forceinline__ void compute_page(WaveState<GQ> &W, unsigned char *st
             for (int a = 0; a < 4; ++a)
                 mx = fmaxf(mx, sv[cb][a]);
         // scores are sv - Y: the max over the row and the exponents absorb Y
-        const float yk = (GQ == 16 ? Yt[ri] : Yt[ri] + Yt[ri + 1]) * W.qk_c;
+        const float yk = (GQ == 16 ? Yt[ri] : Yt[ri] + Yt[ri + 1]) * W.qk_c[0];
         mx = row_max16(mx) - yk;
         const float mn = fmaxf(W.m_run[j], mx);
         alpha[j] = __builtin_amdgcn_exp2f(W.m_run[j] - mn);
@@ -666,8 +904,13 @@ __device__ __forceinline__ SegSetup load_setup(const DecodeParams &p, int b, int
 // q halves, the high-bit rows' q values and channels, the tr8 offsets and
 // the score scale.  scratch: LDS the wave may overwrite (256 + GQ * 256 B),
 // free again on return.
-template <int GQ>
-__device__ __forceinline__ void qk_setup(WaveState<GQ> &W, const DecodeParams &p, int b, int kh, const SegSetup &su,
+//
+// bf16: q of a head enters as q 2^(9 - E) in fp16, 2^E the power of two just
+// above its largest |q| (exact for every channel within 2^-23 of that), and
+// the scores take 2^(E - 9) back: with page scales below 16 the operands stay
+// below 2^13, 2^15 on the high-bit rows.
+template <int GQ, bool BF>
+__device__ __forceinline__ void qk_setup(WaveState<GQ, BF> &W, const DecodeParams &p, int b, int kh, const SegSetup &su,
                                          unsigned char *scratch, int lane, int Dk)
 {
     constexpr int ROWS_PER_HEAD = 16 / GQ;
@@ -703,9 +946,43 @@ __device__ __forceinline__ void qk_setup(WaveState<GQ> &W, const DecodeParams &p
     // keeps fp16 products finite up to |q s_k| < 2^19 (2^17 on the high-bit
     // rows, whose q is also multiplied by 4).
     W.prow = hr;
-    W.qk_c = p.sm_scale * kLog2e * kQInv;
     const bool qk_row = GQ == 16 || (r % ROWS_PER_HEAD) < 2;
-    {
+    if constexpr (BF) {
+        unsigned mag = 0;   // largest |q| of MFMA row r's head, as bits
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                mag = max(mag, max(su.qraw[s][j] << 16 & 0x7fffffffu, su.qraw[s][j] & 0x7fff0000u));
+        mag = max(mag, (unsigned)__shfl_xor((int)mag, 16));
+        mag = max(mag, (unsigned)__shfl_xor((int)mag, 32));
+        const int E = (int)(mag >> 23) - 126;
+#pragma unroll
+        for (int j = 0; j < GQ / 4; ++j)   // head slot j of this lane: MFMA row (q HPL + j) ROWS_PER_HEAD
+            W.qk_c[j] = __builtin_amdgcn_ldexpf(p.sm_scale * kLog2e, __shfl(E, (q * (GQ / 4) + j) * ROWS_PER_HEAD) - 9);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            W.hch[i] = rank_chan[8 * q + i];
+        const uint16_t *qrow = p.q + b * p.q_s_seq + q_head(p, kh, hr) * p.q_s_head;
+        const uint16_t *q16 = (const uint16_t *)q_lds;
+        const int pre = 9 - E;
+        float qh[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            qh[i] = __builtin_amdgcn_ldexpf(bf2f(GQ <= 8 ? q16[hr * 128 + W.hch[i]] : qrow[W.hch[i]]), pre + 2);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                W.qv[s][j] = qk_row ? pack_h2(__builtin_amdgcn_ldexpf(bf_lo(su.qraw[s][j]), pre),
+                                              __builtin_amdgcn_ldexpf(bf_hi(su.qraw[s][j]), pre)) : 0u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int r0 = 8 * q + 2 * j;
+            W.qvh[j] = qk_row ? pack_h2(r0 < Dk ? qh[2 * j] : 0.0f, r0 + 1 < Dk ? qh[2 * j + 1] : 0.0f) : 0u;
+        }
+    } else {
+        W.qk_c[0] = p.sm_scale * kLog2e * kQInv;
         const u32x4 *qraw = su.qraw;
 #pragma unroll
         for (int i = 0; i < 8; ++i)
@@ -745,7 +1022,7 @@ __device__ __forceinline__ void qk_setup(WaveState<GQ> &W, const DecodeParams &p
 // holds query head kh * GQ + h.  A page count outside [0, max_pages] or a
 // page id outside the pool makes the partial NaN; no pages leave an empty
 // partial (m = -inf, l = 0, O = 0).
-template <int GQ>
+template <int GQ, bool BF>
 __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned char *stage0, unsigned char *stage1,
                                              int b, int kh, int np_raw, int p0, int p1, int64_t t, const SegSetup &su)
 {
@@ -769,8 +1046,8 @@ __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned cha
     else if (p1 > np_raw)
         p1 = np_raw;
 
-    WaveState<GQ> W;
-    qk_setup<GQ>(W, p, b, kh, su, stage1, lane, Dk);
+    WaveState<GQ, BF> W;
+    qk_setup<GQ, BF>(W, p, b, kh, su, stage1, lane, Dk);
     // tr4 offsets of value rows R = 32q + 16k + r (GQA 4): 16-byte chunk c of
     // row R sits at 32 R + 16 (c ^ ((R >> 3) & 1)) in the stage.
 #pragma unroll
@@ -790,6 +1067,15 @@ __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned cha
 #pragma unroll
         for (int a = 0; a < 4; ++a)
             W.O[cb][a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (BF) {
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+#pragma unroll
+                for (int j = 0; j < HPL; ++j)
+                    W.ob[cb][a][j] = 0.0f;
+    }
 #pragma unroll
     for (int ch = 0; ch < 4; ++ch)
         W.o4[ch][0] = W.o4[ch][1] = 0.0f;
@@ -839,7 +1125,7 @@ __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned cha
                 wait_vmcnt<kLoadsPerPage>();
             else
                 wait_vmcnt<0>();
-            compute_page<GQ>(W, stage0, lane, Dk);
+            compute_page<GQ, BF>(W, stage0, lane, Dk);
             if (!next)
                 break;
         }
@@ -858,7 +1144,7 @@ __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned cha
                 wait_vmcnt<kLoadsPerPage>();
             else
                 wait_vmcnt<0>();
-            compute_page<GQ>(W, stage1, lane, Dk);
+            compute_page<GQ, BF>(W, stage1, lane, Dk);
         }
     }
     if (poison)
@@ -871,7 +1157,7 @@ __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned cha
         const int h = q * HPL + j;
         const int64_t row = t * GQ + h;
         float *o = p.ws_o + row * 128;
-        if constexpr (GQ == 4) {
+        if constexpr (GQ == 4 && !BF) {
             // o4[ch][e] is O of channel 32ch + 2r + e
 #pragma unroll
             for (int ch = 0; ch < 4; ++ch) {
@@ -887,6 +1173,8 @@ __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned cha
                 float4 v = make_float4(W.O[cb][0][j * RSTEP] * kSub, W.O[cb][1][j * RSTEP] * (kSub * 0.25f),
                                        W.O[cb][2][j * RSTEP] * (kSub * 0.0625f),
                                        W.O[cb][3][j * RSTEP] * (kSub * 0.015625f));
+                if constexpr (BF)
+                    v = make_float4(W.ob[cb][0][j], W.ob[cb][1][j], W.ob[cb][2][j], W.ob[cb][3][j]);
                 if (poison)
                     v = make_float4(__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""));
                 *(float4 *)(o + 64 * cb + 4 * r) = v;
@@ -996,7 +1284,7 @@ __device__ __forceinline__ DecodeParams kernel_params(KernargParams pp)
 // pair.  Steps do not cross from sinks into key-only pages, nor out of one.
 // Returns each head's (m, l) and O (channels 2 lane, 2 lane + 1); m is NaN
 // if a key-only page id lies outside the pool.
-template <int GQ>
+template <int GQ, bool BF>
 __device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int hi, unsigned char *kst,
                               unsigned char *vst, float *m_out, float *l_out, float (*O)[2])
 {
@@ -1060,27 +1348,29 @@ __device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int 
                     c0 = min(hi, kbeg + 128 * (pg + 1));
                     continue;
                 }
-                WaveState<GQ> W;
+                WaveState<GQ, BF> W;
                 const SegSetup su = load_setup<GQ>(p, b, kh, L.npv + pg, L.npv + pg + 1);
-                qk_setup<GQ>(W, p, b, kh, su, vst, lane, p.Dk);
+                qk_setup<GQ, BF>(W, p, b, kh, su, vst, lane, p.Dk);
                 issue_page(kst, page_src(p, (int64_t)page * p.Hkv + kh), lane, p.Dk);
                 wait_vmcnt<0>();
                 f32x4 Sp[2][4], Yt;
-                page_qk<GQ>(W, kst, lane, p.Dk, Sp, Yt);
+                float kmul;
+                page_qk<GQ, BF>(W, kst, lane, p.Dk, Sp, Yt, kmul);
                 const int q = kq;
                 float *scw = (float *)kst;
 #pragma unroll
                 for (int j = 0; j < HPL; ++j) {
                     const int ri = j * RSTEP;
                     // the page path's scale (its operand carries 2^-3 q)
-                    const float yk = (GQ == 16 ? Yt[ri] : Yt[ri] + Yt[ri + 1]) * W.qk_c;
+                    const float page_c = BF ? W.qk_c[BF ? j : 0] * kmul : W.qk_c[0];
+                    const float yk = (GQ == 16 ? Yt[ri] : Yt[ri] + Yt[ri + 1]) * page_c;
 #pragma unroll
                     for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
                         for (int a = 0; a < 4; ++a)
                             scw[(q * HPL + j) * 128 + 64 * cb + 4 * r + a] =
                                 (GQ == 16 ? Sp[cb][a][ri] : Sp[cb][a][ri] + Sp[cb][a][ri + 1]) *
-                                    (W.qk_c * (kSub / (float)(1 << (2 * a)))) - yk;
+                                    (page_c * (kSub / slot_weight<BF>(a))) - yk;
                 }
                 __syncthreads();  // scores in kst before they are read back
                 page_in_kst = pg;
@@ -1124,7 +1414,10 @@ __device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int 
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
                     const half8 kb = *(const half8 *)(kst + 256 * n + 16 * ((4 * s + kq) ^ r));
-                    S[tg] = mfma(qa[s], kb, S[tg]);
+                    if constexpr (BF)
+                        S[tg] = mfma_bf(__builtin_bit_cast(bf16x8, qa[s]), __builtin_bit_cast(bf16x8, kb), S[tg]);
+                    else
+                        S[tg] = mfma(qa[s], kb, S[tg]);
                 }
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -1172,8 +1465,8 @@ __device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int 
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const half2v h = as_h2(vv[e]);
-                    O[g][0] += wt[e] * (float)h[0];
-                    O[g][1] += wt[e] * (float)h[1];
+                    O[g][0] += wt[e] * (BF ? bf_lo(vv[e]) : (float)h[0]);
+                    O[g][1] += wt[e] * (BF ? bf_hi(vv[e]) : (float)h[1]);
                 }
             }
         }
@@ -1191,7 +1484,7 @@ __device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int 
 
 // FP16 tokens [lo, hi) of pair (b, kh) as partial t.  Out of line: the page
 // loop's registers need not be kept around it.
-template <int GQ>
+template <int GQ, bool BF>
 __device__ __forceinline__ void fp16_partial(KernargParams kp, int b, int kh, int lo, int hi, int64_t t,
                                           unsigned char *stage0, unsigned char *stage1)
 {
@@ -1205,7 +1498,7 @@ __device__ __forceinline__ void fp16_partial(KernargParams kp, int b, int kh, in
     hi = __builtin_amdgcn_readfirstlane(hi);
     const int lane = threadIdx.x;
     float m[GQ], l[GQ], O[GQ][2];
-    fp16_segments<GQ>(P, b, kh, lo, hi, stage0, stage1, m, l, O);
+    fp16_segments<GQ, BF>(P, b, kh, lo, hi, stage0, stage1, m, l, O);
     for (int g = 0; g < GQ; ++g) {
         const int64_t row = t * GQ + g;
         *(float2 *)(P.ws_o + row * 128 + 2 * lane) = make_float2(O[g][0], O[g][1]);
@@ -1225,7 +1518,7 @@ __device__ __forceinline__ void fp16_partial(KernargParams kp, int b, int kh, in
 // plan: a run of pages or of FP16 tokens of one pair per segment, one
 // partial per segment.  w is the workgroup's XCD-local order
 // (xcd_local_index), so the consecutive waves of a pair share an XCD and its L2.
-template <int GQ>
+template <int GQ, bool BF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(GQ <= 8 ? 2 : 1)))
 void decode_mfma_kernel(DecodeParams p)
 {
@@ -1349,7 +1642,7 @@ void decode_mfma_kernel(DecodeParams p)
             else
                 su = load_setup<GQ>(P, sq.b, kh, p0, p1);
             use_spec = false;
-            page_segment<GQ>(P, stage0, stage1, sq.b, kh, sq.np_raw, p0, p1, (int64_t)w + 2 * j, su);
+            page_segment<GQ, BF>(P, stage0, stage1, sq.b, kh, sq.np_raw, p0, p1, (int64_t)w + 2 * j, su);
             if (e == u_end && F > 0 && e == s_j + sq.npu)
                 empty_partial<GQ>(P, (int64_t)w + 2 * j + 1);
             u = e;
@@ -1358,7 +1651,7 @@ void decode_mfma_kernel(DecodeParams p)
             const int64_t e = min(u_end, s_j + per_pair);
             const int fa = (int)(off - sq.npu), fc = (int)(e - s_j - sq.npu);
             const int ntok = seq_tokens(kernel_params(kp), sq.b);  // the tokens the F units share
-            fp16_partial<GQ>(kp, sq.b, kh, fa * ntok / F, fc * ntok / F, (int64_t)w + 2 * j + 1, stage0, stage1);
+            fp16_partial<GQ, BF>(kp, sq.b, kh, fa * ntok / F, fc * ntok / F, (int64_t)w + 2 * j + 1, stage0, stage1);
             u = e;
         }
         if (u == s_j + per_pair && lane == 0)  // this wave ends the pair: its last partial
@@ -1384,7 +1677,7 @@ static bool seg_aligned(const kitty_fp16_seg &s)
 bool mfma_shape_supported(const DecodeParams &p)
 {
     return p.D == 128 && p.G == 128 && p.Dk >= 0 && p.Dk <= 32 && (p.GQ == 4 || p.GQ == 8 || p.GQ == 16) &&
-           !p.meta_bf16 && !p.act_bf16;
+           p.meta_bf16 == p.act_bf16;
 }
 
 bool mfma_path_supported(const DecodeParams &p)
@@ -1396,13 +1689,22 @@ bool mfma_path_supported(const DecodeParams &p)
            ((uintptr_t)p.value & 15) == 0 && ((uintptr_t)p.value_meta & 15) == 0;
 }
 
+template <int GQ>
+static void launch_group(const DecodeParams &p, hipStream_t stream)
+{
+    const dim3 grid((unsigned)p.page_waves);
+    if (p.act_bf16)
+        hipLaunchKernelGGL((decode_mfma_kernel<GQ, true>), grid, dim3(64), 0, stream, p);
+    else
+        hipLaunchKernelGGL((decode_mfma_kernel<GQ, false>), grid, dim3(64), 0, stream, p);
+}
+
 int launch_mfma(const DecodeParams &p, hipStream_t stream)
 {
-    dim3 grid((unsigned)p.page_waves);
     switch (p.GQ) {
-    case 4: hipLaunchKernelGGL(decode_mfma_kernel<4>, grid, dim3(64), 0, stream, p); break;
-    case 8: hipLaunchKernelGGL(decode_mfma_kernel<8>, grid, dim3(64), 0, stream, p); break;
-    case 16: hipLaunchKernelGGL(decode_mfma_kernel<16>, grid, dim3(64), 0, stream, p); break;
+    case 4: launch_group<4>(p, stream); break;
+    case 8: launch_group<8>(p, stream); break;
+    case 16: launch_group<16>(p, stream); break;
     default: return fail(KITTY_E_UNSUPPORTED, "MFMA decode needs a GQA group of 4, 8 or 16");
     }
     return check_launch("decode_mfma_kernel");

@@ -280,10 +280,12 @@ class DecodePlan:
     tail_k/v (B, Hkv, T, D) fp16 + tail_len (B,) int32; out (B, Hq, D) fp16.
     With a bfloat16 config, q, the sinks and the tails are bfloat16 and so
     are the metadata pools; out stays fp16 (the reference returns fp16,
-    kernels/attention.py:189).  ``kernel`` names the split kernel the plan
-    runs ("mfma" or "generic"); a plan at the production shape that falls
-    back to the generic kernel (repeated boost ranks, bf16 or misaligned
-    buffers) warns once per process.
+    kernels/attention.py:189).  ``kernel`` is "mfma" where the float16 MFMA
+    split kernel runs and "generic" for everything else: the shape-generic
+    kernel and, at the production shape with bfloat16 throughout, the bfloat16
+    instance of the MFMA kernel, which keeps the generic kernel's fp32
+    accuracy.  A production-shape plan that is not "mfma" (repeated boost
+    ranks, bf16 or misaligned buffers) warns once per process.
 
     Independent value stream (the KIVI split of the pipeline's FP16 value
     window): num_pages_v (B,) int32 value pages and tail_len_v (B,) int32
@@ -412,8 +414,13 @@ def _warn_generic(boost_unique: bool, act_dtype: int, meta_dtype: int) -> None:
     _warned_generic = True
     if not boost_unique:
         why = "a boost_idx row repeats a rank below d_boost"
+    elif act_dtype == _hip.KITTY_DTYPE_BF16 and meta_dtype == _hip.KITTY_DTYPE_BF16:
+        warnings.warn("kitty paged decode runs outside the float16 MFMA path because the buffers are bfloat16: the "
+                      "bfloat16 instance of the MFMA kernel where buffers and pools are 16-byte aligned, else the "
+                      "shape-generic kernel", RuntimeWarning, stacklevel=3)
+        return
     elif act_dtype == _hip.KITTY_DTYPE_BF16 or meta_dtype == _hip.KITTY_DTYPE_BF16:
-        why = "the buffers are bfloat16"
+        why = "only some of the buffers are bfloat16"
     else:
         why = "a pool or FP16 buffer is not 16-byte aligned"
     warnings.warn(f"kitty paged decode runs the shape-generic kernel because {why}; at this shape it is about "
