@@ -41,7 +41,8 @@ static int fp16_weight(int GQ)
 {
     return GQ <= 4 ? KITTY_FP16_WEIGHT_GQ4 : (GQ <= 8 ? KITTY_FP16_WEIGHT_GQ8 : KITTY_FP16_WEIGHT_GQ16);
 }
-constexpr int kMinChunk = 4;  // fewest units per wave of the unit-balanced plan
+constexpr int kMinChunk = 4;  // units per wave of the unit-balanced plan before every resident slot works
+constexpr int kChunkLo = 2;   // and while at most one wave per SIMD does (plan_waves)
 
 // Split size of the uniform plan (generic kernel).  Every (b, kh) pair gets
 // n_splits page splits plus one FP16 split; when the batch allows it, the
@@ -71,23 +72,27 @@ static void set_plan(DecodeParams &p, const kitty_decode_args &a, bool balanced)
     if (!balanced) {
         p.pages_per_split = choose_pages_per_split(a, p.n_fp16);
         p.n_splits = (a.max_pages + p.pages_per_split - 1) / p.pages_per_split;
-        p.page_waves = p.min_chunk = p.fp16_weight = p.fp16_units = 0;
+        p.page_waves = p.simd_waves = p.chunk_lo = p.min_chunk = p.fp16_weight = p.fp16_units = p.static_waves = 0;
         return;
     }
     p.pages_per_split = p.n_splits = 0;
     p.fp16_weight = fp16_weight(p.GQ);
     p.fp16_units = seq_fp16_units(p.sink_cap + p.tail_v_cap, p.fp16_weight);
     const int64_t res = resident_waves(p.GQ <= 8 ? 8 : 4);
+    p.simd_waves = (int)resident_waves(4);
     if (a.pages_per_split > 0) {
-        p.min_chunk = a.pages_per_split;
+        p.chunk_lo = p.min_chunk = a.pages_per_split;
         const int64_t pairs = (int64_t)a.batch * a.num_kv_heads;
         const int64_t umax = (int64_t)a.max_pages + p.fp16_units + 1;
         const int64_t waves = pairs * ((umax + p.min_chunk - 1) / p.min_chunk);
         p.page_waves = (int)(waves < 1 ? 1 : (waves > 16 * res ? 16 * res : waves));
     } else {
+        p.chunk_lo = kChunkLo;
         p.min_chunk = kMinChunk;
         p.page_waves = (int)res;  // every resident slot (fewer waves measured slower)
     }
+    const int64_t units = (int64_t)seq_page_units(a.max_pages, a.max_pages, p.fp16_units) + p.fp16_units;
+    p.static_waves = plan_waves((int64_t)a.batch * a.num_kv_heads * units, p.page_waves, p.simd_waves, p.chunk_lo, p.min_chunk);
 }
 
 static void sub_group(DecodeParams &p, const kitty_decode_args &a, int s);

@@ -45,10 +45,11 @@ struct DecodeParams {
     int act_bf16;  // q, sinks and tails hold bf16 (else fp16)
     float sm_scale;
     // Unit-balanced plan of the MFMA kernel (balanced = 1): the grid has
-    // page_waves waves, each at least min_chunk units; fp16_weight = units
+    // page_waves waves (plan_waves says how many work); fp16_weight = units
     // charged per 128 sink + tail tokens.
-    int balanced, page_waves, min_chunk, fp16_weight;
+    int balanced, page_waves, simd_waves, chunk_lo, min_chunk, fp16_weight;
     int fp16_units;  // FP16 units per pair: seq_fp16_units(sink_cap + tail_v_cap, fp16_weight)
+    int static_waves;  // plan_waves of the batch with every sequence at max_pages
     float *ws_o;  // uniform: [B][Hq][num_partials][D]; balanced: [partial t][GQ][D]
     float *ws_ml; // the same rows: running max (log2 domain) and sum
     int *ws_pair; // balanced: [B * Hkv][2] first and last partial t of each (b, kh)
@@ -134,13 +135,38 @@ __host__ __device__ inline int seq_fp16_units(int ntok, int weight)
     return ntok > 0 ? (int)(((int64_t)ntok * weight + 127) / 128) : 0;
 }
 
-// working waves for U units: at most page_waves, each at least min_chunk units
-__host__ __device__ inline int plan_waves(int64_t U, int page_waves, int min_chunk)
+// Working waves for U units: page_waves once each has min_chunk units.  Below
+// that, min_chunk units per wave, but down to chunk_lo while that leaves at most
+// one wave per SIMD (simd_waves): a wave's units run one after the other, two
+// of them (32 FP16 tokens, one memory round trip) being the shortest chain,
+// and a second wave on a SIMD slows both.  Measured, decode of fp16 batches of 8
+// KV heads, chunks of 4 / 3 / 2 / 1 units: 1 x 1,024 tokens (192 units) 16.1 /
+// 13.8 / 14.0 / 14.4 us, 8 x 1,024 (1,600) 18.0 / 15.6 / 15.8 / 17.8, 8 x 4,096
+// (3,136) 19.5 / 19.1 / 19.8 / 26.4, 16 x 4,096 (6,272) 24.3 / 27.7 / 29.9 / 40.6
+// (before: always 4).  The default plan of 8 x 4,096 tokens took 24.4 us with its
+// 784 waves on the first three XCDs and takes 17.3 us on all eight (plan_wave_of).
+__host__ __device__ inline int plan_waves(int64_t U, int page_waves, int simd_waves, int chunk_lo, int min_chunk)
 {
     if (U >= (int64_t)page_waves * min_chunk)
         return page_waves;
-    const int w = (int)((uint32_t)U / (uint32_t)min_chunk);  // U < 2^31 here
-    return w < 1 ? 1 : w;
+    const uint32_t u = (uint32_t)U;  // U < 2^31 here
+    uint32_t chunk = (u + (uint32_t)simd_waves - 1) / (uint32_t)simd_waves;
+    chunk = chunk < (uint32_t)chunk_lo ? chunk_lo : (chunk > (uint32_t)min_chunk ? min_chunk : chunk);
+    const int w = (int)(u / chunk);
+    return w < 1 ? 1 : (w > page_waves ? page_waves : w);
+}
+
+// Wave of the plan that workgroup i of n runs, W of them working (W <= n): the
+// XCDs (workgroup i runs on XCD i % 8) each take an eighth of the plan's
+// consecutive waves, so work that shares data shares an L2 and a plan of few
+// waves still uses every XCD.  W or more: the workgroup has no work.
+__host__ __device__ inline int plan_wave_of(int i, int n, int W)
+{
+    if (n % 8)
+        return i;
+    const unsigned x = (unsigned)i & 7u, lo = (unsigned)W * x >> 3, hi = (unsigned)W * (x + 1) >> 3;  // W < 2^20
+    const unsigned w = lo + ((unsigned)i >> 3);
+    return (int)(w < hi ? w : (unsigned)W);
 }
 
 // Workgroup i of a launch runs on XCD i % 8 (each XCD has its own L2).  When

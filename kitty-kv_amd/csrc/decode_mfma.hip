@@ -1517,7 +1517,7 @@ __device__ __forceinline__ void fp16_partial(KernargParams kp, int b, int kh, in
 // Wave w works through units [w U / W, (w + 1) U / W) of the unit-balanced
 // plan: a run of pages or of FP16 tokens of one pair per segment, one
 // partial per segment.  w is the workgroup's XCD-local order
-// (xcd_local_index), so the consecutive waves of a pair share an XCD and its L2.
+// (plan_wave_of), so the consecutive waves of a pair share an XCD and its L2.
 template <int GQ, bool BF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(GQ <= 8 ? 2 : 1)))
 void decode_mfma_kernel(DecodeParams p)
@@ -1529,7 +1529,6 @@ void decode_mfma_kernel(DecodeParams p)
 
     const int lane = threadIdx.x;
     const KernargParams kp = (KernargParams)__builtin_amdgcn_kernarg_segment_ptr();
-    const int w = xcd_local_index(blockIdx.x, gridDim.x);
     const int F = p.fp16_units;
     // ---- the plan's input, page counts 64 sequences per step (issued first)
     int np_l = 0, units_l = 0;  // sequence b0 + lane of the current step
@@ -1545,13 +1544,14 @@ void decode_mfma_kernel(DecodeParams p)
     const int units_s = seq_page_units(p.max_pages, p.max_pages, F) + F;
     const int npu_s = units_s - F;
     const int64_t U_s = (int64_t)p.B * p.Hkv * units_s;
-    const int W_s = plan_waves(U_s, p.page_waves, p.min_chunk);
+    const int W_s = p.static_waves;
+    int w = plan_wave_of(blockIdx.x, gridDim.x, W_s);
     int64_t s0 = 0, s1 = 0;
     int g_j = 0;
     bool g_page = false;
     if (w < W_s) {
         wave_units(U_s, W_s, w, s0, s1);
-        g_j = (int)((uint64_t)s0 / (uint32_t)units_s);
+        g_j = U_s <= 0xffffffffll ? (int)((uint32_t)s0 / (uint32_t)units_s) : (int)((uint64_t)s0 / (uint32_t)units_s);
         g_page = s0 - (int64_t)g_j * units_s < npu_s;
     }
     const int g_b = g_j / p.Hkv, g_kh = g_j - g_b * p.Hkv;
@@ -1591,7 +1591,8 @@ void decode_mfma_kernel(DecodeParams p)
             tot += __builtin_amdgcn_readlane(wave_incl_scan(units_l, lane), 63);
         }
         U = tot * p.Hkv;
-        W = plan_waves(U, p.page_waves, p.min_chunk);
+        W = plan_waves(U, p.page_waves, p.simd_waves, p.chunk_lo, p.min_chunk);
+        w = plan_wave_of(blockIdx.x, gridDim.x, W);
         if (w >= W)
             return;
         int64_t u_end;
