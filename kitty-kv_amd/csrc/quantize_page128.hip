@@ -24,6 +24,12 @@
 // a zero row instead of branching, and the destination page id is looked up
 // after the loads are issued.
 //
+// bf16 blocks take the same path on fp32 copies of their elements (exact): the
+// ranges with fp32 min / max, which skip NaN elements as the shape-generic
+// kernel's comparisons do, the partials between lanes and waves packed back to
+// bf16.  512 pages x 8 heads of keys and values: 81 us, where the shape-generic
+// kernel that bf16 ran before took 741 (fp16: 64).
+//
 // Arithmetic is that of quantize.h (bit-exact with the reference).  The
 // zero points use the multiply-by-reciprocal of rint_quot below, which
 // returns the same integer as rint of the correctly rounded quotient; the
@@ -36,7 +42,6 @@
 namespace kitty {
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / 64;
@@ -52,8 +57,6 @@ constexpr int kRedOff = kHighOff + 128 * 32;            // key partial min / max
 constexpr int kParOff = kRedOff + 2 * kWaves * 128 * 2; // parameters: s, 1/s, z, mq, high row: 5 x 128 x 4 B
 constexpr int kLdsBytes = kParOff + 5 * 128 * 4;        // 15,104
 
-__device__ __forceinline__ h2 as_h2(unsigned w) { return __builtin_bit_cast(h2, w); }
-__device__ __forceinline__ unsigned as_u(h2 v) { return __builtin_bit_cast(unsigned, v); }
 // Packed fp16 min / max as single instructions.  The builtins' IEEE minnum
 // first quiets each operand that may be a signalling NaN (a v_pk_max_f16
 // x, x per bit-cast operand, about 200 in this kernel); the inputs here are
@@ -77,14 +80,53 @@ __device__ __forceinline__ unsigned pk_min_neg(unsigned a, unsigned b)
     asm("v_pk_min_f16 %0, %1, %2 neg_lo:[1,1] neg_hi:[1,1]" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
-__device__ __forceinline__ h2 hmin(h2 a, h2 b) { return as_h2(pk_min(as_u(a), as_u(b))); }
-__device__ __forceinline__ h2 hmax(h2 a, h2 b) { return as_h2(pk_max(as_u(a), as_u(b))); }
+__device__ __forceinline__ float bf_lo(unsigned w) { return __builtin_bit_cast(float, w << 16); }
+__device__ __forceinline__ float bf_hi(unsigned w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
+// two fp32 values that bf16 holds exactly, packed (a low)
+__device__ __forceinline__ unsigned bf_pack(float a, float b)
+{
+    return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x07060302u);
+}
 
-__device__ __forceinline__ _Float16 chan(const u32x4 &v, int c)
+// Packed min / max of two 16-bit elements.  bf16: through fp32, a NaN giving
+// way to the other operand.
+template <bool BF>
+__device__ __forceinline__ unsigned min2(unsigned a, unsigned b)
+{
+    if constexpr (BF)
+        return bf_pack(__builtin_fminf(bf_lo(a), bf_lo(b)), __builtin_fminf(bf_hi(a), bf_hi(b)));
+    else
+        return pk_min(a, b);
+}
+template <bool BF>
+__device__ __forceinline__ unsigned max2(unsigned a, unsigned b)
+{
+    if constexpr (BF)
+        return bf_pack(__builtin_fmaxf(bf_lo(a), bf_lo(b)), __builtin_fmaxf(bf_hi(a), bf_hi(b)));
+    else
+        return pk_max(a, b);
+}
+
+template <bool BF>
+__device__ __forceinline__ float elem_f(uint16_t b)
+{
+    return BF ? bf2f(b) : h2f(b);
+}
+
+// Element c of a thread's 8: _Float16 (read in place by v_fma_mix_f32) or fp32.
+template <bool BF>
+__device__ __forceinline__ auto chan(const u32x4 &v, int c)
 {
     const unsigned w = v[c >> 1];
-    return __builtin_bit_cast(_Float16, (uint16_t)((c & 1) ? (w >> 16) : (w & 0xffffu)));
+    if constexpr (BF)
+        return (c & 1) ? bf_hi(w) : bf_lo(w);
+    else
+        return __builtin_bit_cast(_Float16, (uint16_t)((c & 1) ? (w >> 16) : (w & 0xffffu)));
 }
+
+// Scales whose reciprocal v_rcp_f32 may flush (bf16 blocks only: fp16 ranges
+// end at 2^17): the quotients are computed exactly there.
+constexpr float kRcpMax = 0x1p125f;
 
 // A lane permutation within rows of 16 (every lane has a source, so no old
 // value is needed).
@@ -102,12 +144,14 @@ __device__ __forceinline__ unsigned dpp(unsigned v)
 // recomputed exactly (about 1 element in 8,000 for smooth data; every tie of
 // grid-aligned data).  For |x / s| >= 32 both round outside [-mq, mq] with
 // the same sign, and the code / zero-point clamps give the same end value.
-// Inputs are finite fp16.
+// Inputs are finite fp16, or bf16 of any value (an infinite scale makes every
+// quotient 0 or NaN, here as in the division).
+template <bool BF>
 __device__ __forceinline__ float rint_quot(float x, float s, float rs)
 {
     const float y = x * rs;
     float n = __builtin_rintf(y);
-    if (__builtin_expect(__builtin_fabsf(y - n) > 0.5f - 0x1p-14f, 0))
+    if (__builtin_expect(__builtin_fabsf(y - n) > 0.5f - 0x1p-14f || (BF && s >= kRcpMax), 0))
         n = __builtin_rintf(x / s);
     return n;
 }
@@ -127,8 +171,8 @@ __device__ __forceinline__ float rint_quot(float x, float s, float rs)
 // is the clamped code of rint(q) + z <= 0; at or above 2^24, p + z >= 2^23
 // and t clamps to mq, as does rint(q) + z.  Outside |q| < 32 the clamped
 // codes agree for the same reason as in rint_quot.  A group with an element
-// near a half-integer recomputes all eight from the correctly rounded
-// quotient.  The fp16 operands are read in place (v_fma_mix_f32).
+// near a half-integer looks at its eight again and recomputes those near one
+// from the correctly rounded quotient (magic_exact).  The fp16 operands are read in place (v_fma_mix_f32).
 //
 // The kernels run the fast step of all groups of a thread first and the
 // (rarely taken) exact recomputations after.
@@ -178,15 +222,19 @@ __device__ __forceinline__ void magic_fast(X x, RS rs, CZ cz, float (&t)[NG][8],
     }
 }
 
-// Exact step for a group whose dev exceeds kNearHalf.
-__device__ __forceinline__ void magic_exact8(const _Float16 (&x)[8], float s, float cz, float (&t)[8])
+// Exact step for an element of a group whose dev exceeds kNearHalf: only
+// elements near a half-integer themselves are divided (bf16 blocks, whose
+// elements and ranges lie on coarse grids, have exact ties in most waves: 512
+// pages x 8 heads took 91 us with the whole group divided, 81 so; fp16 66 and 64).
+template <bool BF>
+__device__ __forceinline__ void magic_exact(float x, float s, float rs, float cz, float &t)
 {
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-        t[e] = __builtin_rintf((float)x[e] / s) + cz;  // cz exact: z is an integer in [0, 15]
+    const float e = __builtin_fmaf(x, rs, -(t - cz));
+    if (__builtin_fabsf(e) > kNearHalf || (BF && s >= kRcpMax))
+        t = __builtin_rintf(x / s) + cz;  // cz exact: z is an integer in [0, 15]
 }
 
-// The clamped code of t from magic_fast / magic_exact8 as the low bits of a word:
+// The clamped code of t from magic_fast / magic_exact as the low bits of a word:
 // kC + clamp(t - kC, 0, mq) has the bit pattern 0x4B000000 | code.
 __device__ __forceinline__ unsigned code_bits(float t, float mq)
 {
@@ -287,7 +335,7 @@ __device__ __forceinline__ void load_tile_channel_major(const uint16_t *src, int
             r[k][j] = __builtin_amdgcn_perm(c[2 * j + 1][k >> 1], c[2 * j][k >> 1], (k & 1) ? 0x07060302u : 0x05040100u);
 }
 
-template <bool CHAN_MAJOR>
+template <bool CHAN_MAJOR, bool BF>
 __device__ void key_block(const QuantLaunch &L, int o, int i, unsigned char *lds)
 {
     const kitty_page_store &st = L.st;
@@ -295,6 +343,7 @@ __device__ void key_block(const QuantLaunch &L, int o, int i, unsigned char *lds
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int cg = lane & 15, tt = wave * 4 + (lane >> 4);
     const int Dk = st.d_boost;
+    const bool mbf = st.meta_dtype == KITTY_DTYPE_BF16;
 
     u32x4 r[kTok];
     if constexpr (CHAN_MAJOR)
@@ -311,29 +360,44 @@ __device__ void key_block(const QuantLaunch &L, int o, int i, unsigned char *lds
     for (int e = tid; e < Dk * 8; e += kThreads)
         high[e] = 0u; // rows with no channel stay 0 (the reference's zeroed tensor)
 
-    // min / max over the thread's tokens, channel pairs packed in fp16 (:76-77)
-    h2 mn[4], mx[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-        mn[j] = mx[j] = as_h2(r[0][j]);
-#pragma unroll
-    for (int k = 1; k < kTok; ++k)
+    // min / max over the thread's tokens, channel pairs packed (:76-77)
+    unsigned mn[4], mx[4];
+    if constexpr (BF) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            mn[j] = hmin(mn[j], as_h2(r[k][j]));
-            mx[j] = hmax(mx[j], as_h2(r[k][j]));
+            float lo[2], hi[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float a = chan<true>(r[0], 2 * j + e), b2 = chan<true>(r[1], 2 * j + e),
+                            c = chan<true>(r[2], 2 * j + e), d = chan<true>(r[3], 2 * j + e);
+                lo[e] = __builtin_fminf(__builtin_fminf(a, b2), __builtin_fminf(c, d));
+                hi[e] = __builtin_fmaxf(__builtin_fmaxf(a, b2), __builtin_fmaxf(c, d));
+            }
+            mn[j] = bf_pack(lo[0], lo[1]);
+            mx[j] = bf_pack(hi[0], hi[1]);
         }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            mn[j] = mx[j] = r[0][j];
+#pragma unroll
+        for (int k = 1; k < kTok; ++k)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                mn[j] = pk_min(mn[j], r[k][j]);
+                mx[j] = pk_max(mx[j], r[k][j]);
+            }
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        mn[j] = hmin(mn[j], as_h2((unsigned)__shfl_xor((int)as_u(mn[j]), 16)));
-        mx[j] = hmax(mx[j], as_h2((unsigned)__shfl_xor((int)as_u(mx[j]), 16)));
-        mn[j] = hmin(mn[j], as_h2((unsigned)__shfl_xor((int)as_u(mn[j]), 32)));
-        mx[j] = hmax(mx[j], as_h2((unsigned)__shfl_xor((int)as_u(mx[j]), 32)));
+        mn[j] = min2<BF>(mn[j], (unsigned)__shfl_xor((int)mn[j], 16));
+        mx[j] = max2<BF>(mx[j], (unsigned)__shfl_xor((int)mx[j], 16));
+        mn[j] = min2<BF>(mn[j], (unsigned)__shfl_xor((int)mn[j], 32));
+        mx[j] = max2<BF>(mx[j], (unsigned)__shfl_xor((int)mx[j], 32));
     }
     if (lane < 16) {  // the wave's partial for channels 8cg..8cg+7
-        *(u32x4 *)(lds + kRedOff + wave * 256 + cg * 16) = u32x4{as_u(mn[0]), as_u(mn[1]), as_u(mn[2]), as_u(mn[3])};
-        *(u32x4 *)(lds + kRedOff + kWaves * 256 + wave * 256 + cg * 16) =
-            u32x4{as_u(mx[0]), as_u(mx[1]), as_u(mx[2]), as_u(mx[3])};
+        *(u32x4 *)(lds + kRedOff + wave * 256 + cg * 16) = u32x4{mn[0], mn[1], mn[2], mn[3]};
+        *(u32x4 *)(lds + kRedOff + kWaves * 256 + wave * 256 + cg * 16) = u32x4{mx[0], mx[1], mx[2], mx[3]};
     }
     __syncthreads();
 
@@ -345,23 +409,27 @@ __device__ void key_block(const QuantLaunch &L, int o, int i, unsigned char *lds
     uint16_t meta_s = 0, meta_z = 0;
     if (tid < 128) {  // channel d = tid
         const uint16_t *rmn = (const uint16_t *)(lds + kRedOff), *rmx = rmn + kWaves * 128;
-        float cmn = h2f(rmn[tid]), cmx = h2f(rmx[tid]);
+        float cmn = elem_f<BF>(rmn[tid]), cmx = elem_f<BF>(rmx[tid]);
 #pragma unroll
         for (int w2 = 1; w2 < kWaves; ++w2) {
-            cmn = __builtin_fminf(cmn, h2f(rmn[w2 * 128 + tid]));
-            cmx = __builtin_fmaxf(cmx, h2f(rmx[w2 * 128 + tid]));
+            cmn = __builtin_fminf(cmn, elem_f<BF>(rmn[w2 * 128 + tid]));
+            cmx = __builtin_fmaxf(cmx, elem_f<BF>(rmx[w2 * 128 + tid]));
+        }
+        if constexpr (BF) {  // a channel of NaNs: the empty range of the generic kernel
+            cmn = __builtin_fminf(cmn, __builtin_inff());
+            cmx = __builtin_fmaxf(cmx, -__builtin_inff());
         }
         const float mq = b < qb.sentinel ? 15.0f : 3.0f;               // :73, 81-82
         const float s = range_of(cmn, cmx) / mq;                       // :78-84
         const float rs = __builtin_amdgcn_rcpf(s);
-        const float z = zp_clamp(rint_quot(-cmn, s, rs), mq);          // :86-87
+        const float z = zp_clamp(rint_quot<BF>(-cmn, s, rs), mq);      // :86-87
         ps[tid] = s;
         prs[tid] = rs;
         pz[tid] = z;
         pmq[tid] = mq;
         phr[tid] = b < Dk ? b : -1;                                    // :113-116
-        meta_s = f2h(s);                                               // :121-122
-        meta_z = f2h(z);
+        meta_s = meta_store(s, mbf);                                   // :121-122
+        meta_z = meta_store(z, mbf);
     }
     __syncthreads();
 
@@ -378,16 +446,16 @@ __device__ void key_block(const QuantLaunch &L, int o, int i, unsigned char *lds
 #pragma unroll
     for (int c = 0; c < 8; ++c)
         cz[c] = kC + z[c];
-    magic_fast<4>([&](int g, int e) { return chan(r[e & 3], 2 * g + (e >> 2)); },
+    magic_fast<4>([&](int g, int e) { return chan<BF>(r[e & 3], 2 * g + (e >> 2)); },
                   [&](int g, int e) { return rs[2 * g + (e >> 2)]; },
                   [&](int g, int e) { return cz[2 * g + (e >> 2)]; }, t, dev);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-        if (__builtin_expect(dev[g] > kNearHalf, 0)) {
+        if (__builtin_expect(dev[g] > kNearHalf || (BF && __builtin_fmaxf(s[2 * g], s[2 * g + 1]) >= kRcpMax), 0)) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const int c = 2 * g + (e >> 2), k = e & 3;
-                t[g][e] = __builtin_rintf((float)chan(r[k], c) / s[c]) + cz[c];
+                magic_exact<BF>((float)chan<BF>(r[k], c), s[c], rs[c], cz[c], t[g][e]);
             }
         }
     }
@@ -418,6 +486,7 @@ __device__ void key_block(const QuantLaunch &L, int o, int i, unsigned char *lds
 
 // ----------------------------------------------------------------- values
 // quantize_value.py:58-90: per token over the 128 channels.
+template <bool BF>
 __device__ void value_block(const QuantLaunch &L, int o, int i, unsigned char *lds)
 {
     const kitty_page_store &st = L.st;
@@ -425,6 +494,7 @@ __device__ void value_block(const QuantLaunch &L, int o, int i, unsigned char *l
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int cg = lane & 15, tt = wave * 4 + (lane >> 4);
 
+    const bool mbf = st.meta_dtype == KITTY_DTYPE_BF16;
     const uint16_t *vsrc = qb.value + outer_offset(qb, o, qb.value_s_seq, qb.value_s_outer) + i * qb.value_s_inner;
     u32x4 r[kTok];
     load_rows(vsrc + 8 * cg, qb.value_s_tok, kTok * tt, qb.value_rows, cg, r);
@@ -437,9 +507,19 @@ __device__ void value_block(const QuantLaunch &L, int o, int i, unsigned char *l
     unsigned mm[kTok];
 #pragma unroll
     for (int k = 0; k < kTok; ++k) {
-        const unsigned a = pk_min(pk_min(r[k][0], r[k][1]), pk_min(r[k][2], r[k][3]));
-        const unsigned b = pk_min(pk_min_neg(r[k][0], r[k][1]), pk_min_neg(r[k][2], r[k][3]));
-        mm[k] = pk_min(__builtin_amdgcn_perm(b, a, 0x05040100u), __builtin_amdgcn_perm(b, a, 0x07060302u));
+        if constexpr (BF) {
+            float lo = chan<true>(r[k], 0), hi = lo;
+#pragma unroll
+            for (int c = 1; c < 8; ++c) {
+                lo = __builtin_fminf(lo, chan<true>(r[k], c));
+                hi = __builtin_fmaxf(hi, chan<true>(r[k], c));
+            }
+            mm[k] = bf_pack(lo, -hi);
+        } else {
+            const unsigned a = pk_min(pk_min(r[k][0], r[k][1]), pk_min(r[k][2], r[k][3]));
+            const unsigned b = pk_min(pk_min_neg(r[k][0], r[k][1]), pk_min_neg(r[k][2], r[k][3]));
+            mm[k] = pk_min(__builtin_amdgcn_perm(b, a, 0x05040100u), __builtin_amdgcn_perm(b, a, 0x07060302u));
+        }
     }
     // ... then over the 16 lanes of the DPP row, as a reduce-scatter: the
     // first two steps pair lane l with a partner (l ^ 15, then l ^ 7), keep
@@ -451,25 +531,29 @@ __device__ void value_block(const QuantLaunch &L, int o, int i, unsigned char *l
     unsigned w[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j)   // row_mirror: l <-> 15 - l
-        w[j] = pk_min(b3 ? mm[j + 2] : mm[j], dpp<0x140>(b3 ? mm[j] : mm[j + 2]));
-    unsigned v = pk_min(b2 ? w[1] : w[0], dpp<0x141>(b2 ? w[0] : w[1]));   // row_half_mirror: l <-> l ^ 7
-    v = pk_min(v, dpp<0x4E>(v));                                           // quad_perm [2,3,0,1]
-    v = pk_min(v, dpp<0xB1>(v));                                           // quad_perm [1,0,3,2]
+        w[j] = min2<BF>(b3 ? mm[j + 2] : mm[j], dpp<0x140>(b3 ? mm[j] : mm[j + 2]));
+    unsigned v = min2<BF>(b2 ? w[1] : w[0], dpp<0x141>(b2 ? w[0] : w[1]));  // row_half_mirror: l <-> l ^ 7
+    v = min2<BF>(v, dpp<0x4E>(v));                                          // quad_perm [2,3,0,1]
+    v = min2<BF>(v, dpp<0xB1>(v));                                          // quad_perm [1,0,3,2]
 
     // lanes 4j of each row: parameters of token 4tt + j
     float *ps = (float *)(lds + kParOff), *prs = ps + 128, *pz = ps + 256;
     if ((cg & 3) == 0) {
-        const float mn = h2f((uint16_t)(v & 0xffffu)), mx = -h2f((uint16_t)(v >> 16));
+        float mn = elem_f<BF>((uint16_t)(v & 0xffffu)), mx = -elem_f<BF>((uint16_t)(v >> 16));
+        if constexpr (BF) {  // a token of NaNs: the empty range of the generic kernel
+            mn = __builtin_fminf(mn, __builtin_inff());
+            mx = __builtin_fmaxf(mx, -__builtin_inff());
+        }
         const float s = range_of(mn, mx) / 3.0f;                       // :65-67
         const float rs = __builtin_amdgcn_rcpf(s);
-        const float z = zp_clamp(rint_quot(-mn, s, rs), 3.0f);         // :69-73
+        const float z = zp_clamp(rint_quot<BF>(-mn, s, rs), 3.0f);     // :69-73
         const int t = kTok * tt + (cg >> 2);
         ps[t] = s;
         prs[t] = rs;
         pz[t] = z;
         const int64_t m = page * st.value_meta_s_page + i * st.value_meta_s_head + 2 * t;
         if (ok)
-            __builtin_nontemporal_store((unsigned)f2h(s) | ((unsigned)f2h(z) << 16),
+            __builtin_nontemporal_store((unsigned)meta_store(s, mbf) | ((unsigned)meta_store(z, mbf) << 16),
                                         (unsigned *)(st.value_scale + m));  // :90, interleaved
     }
     __syncthreads();
@@ -495,16 +579,14 @@ __device__ void value_block(const QuantLaunch &L, int o, int i, unsigned char *l
 #pragma unroll
     for (int k = 0; k < kTok; ++k)
         cz[k] = kC + z[k];
-    magic_fast<kTok>([&](int k, int c) { return chan(r[k], c); }, [&](int k, int) { return rs[k]; },
+    magic_fast<kTok>([&](int k, int c) { return chan<BF>(r[k], c); }, [&](int k, int) { return rs[k]; },
                      [&](int k, int) { return cz[k]; }, t, dev);
 #pragma unroll
     for (int k = 0; k < kTok; ++k) {
-        if (__builtin_expect(dev[k] > kNearHalf, 0)) {
-            _Float16 x[8];
+        if (__builtin_expect(dev[k] > kNearHalf || (BF && s[k] >= kRcpMax), 0)) {
 #pragma unroll
             for (int c = 0; c < 8; ++c)
-                x[c] = chan(r[k], c);
-            magic_exact8(x, s[k], cz[k], t[k]);
+                magic_exact<BF>((float)chan<BF>(r[k], c), s[k], rs[k], cz[k], t[k][c]);
         }
     }
 #pragma unroll
@@ -528,6 +610,7 @@ __device__ void value_block(const QuantLaunch &L, int o, int i, unsigned char *l
     }
 }
 
+template <bool BF>
 __global__ __launch_bounds__(kThreads) void quantize_page128_kernel(QuantLaunch L)
 {
     __shared__ __attribute__((aligned(16))) unsigned char lds[kLdsBytes];
@@ -536,12 +619,12 @@ __global__ __launch_bounds__(kThreads) void quantize_page128_kernel(QuantLaunch 
     if (blockIdx.y == 0) {
         if (L.qb.key) {
             if (L.qb.key_s_chan == 1)
-                key_block<false>(L, o, i, lds);
+                key_block<false, BF>(L, o, i, lds);
             else
-                key_block<true>(L, o, i, lds);
+                key_block<true, BF>(L, o, i, lds);
         }
     } else if (L.qb.value) {
-        value_block(L, o, i, lds);
+        value_block<BF>(L, o, i, lds);
     }
 }
 
@@ -552,8 +635,6 @@ bool page128_supported(const kitty_page_store &st, const kitty_quant_batch &qb)
 {
     if (st.head_dim != 128 || st.page_tokens != 128)
         return false;
-    if (st.meta_dtype != KITTY_DTYPE_F16 || qb.src_dtype != KITTY_DTYPE_F16)
-        return false;  // bf16 blocks or pools: the shape-generic kernel
     if (qb.key) {
         // token-major rows (channel stride 1) or channel-major rows (token stride 1)
         const bool rows = qb.key_s_chan == 1 && mul(qb.key_s_tok, 8);
@@ -587,7 +668,11 @@ bool page128_supported(const kitty_page_store &st, const kitty_quant_batch &qb)
 int launch_page128(const QuantLaunch &L, hipStream_t stream)
 {
     const int64_t nblocks = (int64_t)L.qb.n_outer * L.qb.n_inner;
-    hipLaunchKernelGGL(quantize_page128_kernel, dim3((unsigned)nblocks, 2), dim3(kThreads), 0, stream, L);
+    const dim3 grid((unsigned)nblocks, 2);
+    if (L.qb.src_dtype == KITTY_DTYPE_BF16)
+        hipLaunchKernelGGL(quantize_page128_kernel<true>, grid, dim3(kThreads), 0, stream, L);
+    else
+        hipLaunchKernelGGL(quantize_page128_kernel<false>, grid, dim3(kThreads), 0, stream, L);
     return check_launch("quantize_page128_kernel");
 }
 
