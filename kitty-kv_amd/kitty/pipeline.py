@@ -688,7 +688,8 @@ class KittyInferencePipeline:
             self._block_table[l, sl, :n_full] = pages.view(B, n_full)
             self._pages[slots, l, :n_full] = phys.reshape(B, n_full)
             if R and v_full:
-                pages_v = pages.view(B, n_full)[:, :v_full].reshape(-1)
+                # a copy: one column of the table stays a strided view under reshape
+                pages_v = pages.view(B, n_full)[:, :v_full].contiguous().view(-1)
                 quantize_into_pools(self._store, None, blocks(values, v_full), None, pages_v, cfg.sentinel)
         if rem:
             self._qbuf_k[sl, l, :, :rem] = keys[:, :, n_s + n_full * G:]
