@@ -373,6 +373,51 @@ int kitty_prefill_attention(const kitty_prefill_args *args, kitty_stream_t strea
 #define KITTY_STORE_I32_MAX 320
 int kitty_store_i32(int32_t *const *addrs, const int32_t *values, int32_t n, kitty_stream_t stream);
 
+/* ------------------------------------------------ prompt into the buffers
+ * The FP16 side of a prompt's arrival for B sequences that hold nothing yet
+ * (kitty/attention.py:169-177 pushes its tokens one at a time through
+ * kitty/pipeline.py:115-181), in one launch: of key / value (B, H, T, D) rows
+ * 0 .. n_sink - 1 go to the sink buffers, rows n_sink + key_pages * page_tokens
+ * .. T - 1 to the front of the key buffer, rows n_sink + value_pages *
+ * page_tokens .. T - 1 to the front of the value buffer; the sequences'
+ * block-table entries 0 .. key_pages - 1 are pages[b * key_pages + p] and their
+ * counters (sink fill, key buffer length, key pages, value pages, value buffer
+ * length) those numbers.  Buffers, counters and block table point at the first
+ * sequence's slot; slots follow each other (s_slot, one int32, bt_stride).
+ * The pages themselves are kitty_quantize_kv_blocks'.  Rows 16-byte aligned,
+ * head_dim a multiple of 8, element strides multiples of 8 (ABI version 7). */
+typedef struct {
+    const uint16_t *key, *value;
+    int64_t key_s_seq, key_s_head, key_s_tok, value_s_seq, value_s_head, value_s_tok;
+    uint16_t *sink_k, *sink_v;
+    kitty_slot_layout sink_layout;
+    uint16_t *key_buf;
+    kitty_slot_layout key_layout;
+    uint16_t *value_buf;
+    kitty_slot_layout value_layout;
+    int32_t *counters;       /* sink fill of the first slot; the other four counters_stride int32 apart */
+    int64_t counters_stride;
+    int32_t *block_table;    /* first slot's row */
+    int64_t bt_stride;
+    const int32_t *pages;    /* (B, key_pages), device; unused with no key pages */
+    int32_t batch, num_kv_heads, head_dim, tokens, page_tokens;
+    int32_t n_sink, key_pages, value_pages;
+} kitty_prompt_args;
+
+int kitty_store_prompt(const kitty_prompt_args *args, kitty_stream_t stream);
+
+/* Zeroes n regions (host list; rows of row_bytes, row_stride bytes apart, 4-byte
+ * aligned and sized) in launches of at most KITTY_ZERO_MAX regions: a sequence's
+ * buffers, counters and table when it is reset (kitty/pipeline.py:286-313).
+ * ABI version 7. */
+#define KITTY_ZERO_MAX 16
+typedef struct {
+    void *ptr;
+    int64_t rows, row_bytes, row_stride;
+} kitty_zero_region;
+
+int kitty_zero_regions(const kitty_zero_region *regions, int32_t n, kitty_stream_t stream);
+
 /* ------------------------------------------- sensitivity accumulation
  * Replaces _ChannelAccumulator.update (kitty/sensitivity.py:46-61):
  * out[h*head_dim + d] += sum over b < batch, t < tokens of

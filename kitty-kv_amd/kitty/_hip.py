@@ -118,6 +118,24 @@ class AppendArgs(ctypes.Structure):
     ]
 
 
+class PromptArgs(ctypes.Structure):
+    """kitty_prompt_args: the FP16 rows, table entries and counters of new prompts."""
+    _fields_ = [
+        ("key", _vp), ("value", _vp),
+        ("key_s_seq", _i64), ("key_s_head", _i64), ("key_s_tok", _i64),
+        ("value_s_seq", _i64), ("value_s_head", _i64), ("value_s_tok", _i64),
+        ("sink_k", _vp), ("sink_v", _vp), ("sink_layout", SlotLayout),
+        ("key_buf", _vp), ("key_layout", SlotLayout), ("value_buf", _vp), ("value_layout", SlotLayout),
+        ("counters", _vp), ("counters_stride", _i64), ("block_table", _vp), ("bt_stride", _i64), ("pages", _vp),
+        ("batch", _i32), ("num_kv_heads", _i32), ("head_dim", _i32), ("tokens", _i32), ("page_tokens", _i32),
+        ("n_sink", _i32), ("key_pages", _i32), ("value_pages", _i32),
+    ]
+
+
+class ZeroRegion(ctypes.Structure):
+    _fields_ = [("ptr", _vp), ("rows", _i64), ("row_bytes", _i64), ("row_stride", _i64)]
+
+
 class PrefillArgs(ctypes.Structure):
     """kitty_prefill_args: causal attention of a prompt."""
     _fields_ = [
@@ -138,6 +156,7 @@ EXPORTED_SYMBOLS = (
     "kitty_paged_decode_merge", "kitty_paged_decode_noalloc", "kitty_append_tokens", "kitty_channel_abs_sum",
     "kitty_channel_abs_sum_workspace_size", "kitty_channel_abs_sum_deferred_size", "kitty_channel_abs_sum_deferred",
     "kitty_channel_abs_sum_flush", "kitty_store_i32", "kitty_prefill_attention",
+    "kitty_store_prompt", "kitty_zero_regions",
 )
 
 _lib: Optional[ctypes.CDLL] = None
@@ -176,6 +195,8 @@ def load() -> ctypes.CDLL:
     L.kitty_channel_abs_sum_deferred.argtypes = L.kitty_channel_abs_sum.argtypes
     L.kitty_channel_abs_sum_flush.argtypes = [_vp, _i32, _i32, _vp, _vp]
     L.kitty_store_i32.argtypes = [_vp, _vp, _i32, _vp]
+    L.kitty_store_prompt.argtypes = [ctypes.POINTER(PromptArgs), _vp]
+    L.kitty_zero_regions.argtypes = [ctypes.POINTER(ZeroRegion), _i32, _vp]
     L.kitty_prefill_attention.argtypes = [ctypes.POINTER(PrefillArgs), _vp]
     if L.kitty_abi_version() != KITTY_ABI_VERSION:
         raise ImportError(f"libkitty_hip ABI {L.kitty_abi_version()} != {KITTY_ABI_VERSION}")

@@ -441,28 +441,37 @@ def paged_decode(*args, **kwargs) -> torch.Tensor:
     return decode_plan(*args, **kwargs).run()
 
 
-def prefill_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
-    """True when kitty_prefill_attention takes these (B, heads, T, D) tensors
-    as they are: head_dim 128, one 16-bit dtype, 16-byte rows.  Anything a
-    plain kernel launch would drop stays with torch: inputs that need
-    gradients, forward-mode tangents, functorch transforms, tensor subclasses
-    (fake tensors) and negated or conjugated views."""
-    if not (type(q) is type(k) is type(v) is torch.Tensor and q.device.type == "cuda" and q.device == k.device == v.device):
-        return False
-    if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype:
-        return False
-    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+def plain_rows(*tensors: torch.Tensor) -> bool:
+    """True when a kernel may read these (B, heads, T, D) tensors by pointer:
+    fp16 or bf16 of one dtype on one ROCm device, with 16-byte aligned rows of contiguous
+    channels.  What a plain launch would drop stays with torch: inputs that
+    need gradients, forward-mode tangents, functorch transforms, tensor
+    subclasses (fake tensors) and negated views."""
+    t0 = tensors[0]
+    if t0.device.type != "cuda" or t0.dtype not in (torch.float16, torch.bfloat16):
         return False
     if forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None:
         return False
-    if not (q.dim() == k.dim() == v.dim() == 4 and q.shape[3] == k.shape[3] == 128 and k.shape == v.shape
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) is not torch.Tensor or t.device != t0.device or t.dtype != t0.dtype or t.dim() != 4:
+            return False
+        if (grad and t.requires_grad) or t.is_neg() or t.stride(3) != 1 or t.data_ptr() % 16:
+            return False
+        if any(s % 8 for s in t.stride()[:3]):
+            return False
+    return True
+
+
+def prefill_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """True when kitty_prefill_attention takes these (B, heads, T, D) tensors
+    as they are: plain_rows at head_dim 128."""
+    if not plain_rows(q, k, v):
+        return False
+    if not (q.shape[3] == k.shape[3] == 128 and k.shape == v.shape
             and q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2] and q.shape[2] > 0
             and q.shape[1] > 0 and k.shape[1] > 0 and q.shape[1] % k.shape[1] == 0):
         return False
-    for t in (q, k, v):
-        # a stride of a dimension of size 1 is never used for an address past the row
-        if t.is_neg() or t.stride(3) != 1 or t.data_ptr() % 16 or any(s % 8 for s in t.stride()[:3]):
-            return False
     # 32-bit byte offsets inside a head (kitty_prefill_attention); the launch's grid
     T = q.shape[2]
     return all(0 <= s and (T + 64) * s * 2 + 256 < 1 << 31 for s in (k.stride(2), v.stride(2))) \

@@ -63,7 +63,7 @@ from . import _hip
 from .config import KittyConfig
 from .layout import PageCentricKVLayoutManager
 from .kernels import cpu
-from .kernels.ops import HostStager, QuantizePlan, pool_store, quantize_into_pools
+from .kernels.ops import HostStager, QuantizePlan, plain_rows, pool_store, quantize_into_pools
 
 _FILL, _QLEN, _NPAGES, _NPAGES_V, _VLEN = 0, 1, 2, 3, 4
 
@@ -114,6 +114,8 @@ class KittyInferencePipeline:
         self._slots_of_ids: Dict[Tuple[int, ...], np.ndarray] = {}
         # append arguments per (layer, slots): everything but the token pointers
         self._append_args: Dict[Tuple[int, Tuple[int, ...]], Tuple[_hip.AppendArgs, torch.Tensor]] = {}
+        # per slot: the device regions reset_sequence zeroes
+        self._reset_regions: Dict[int, ctypes.Array] = {}
         self._lib = None
         self._stager = None         # pinned staging rows of _h2d, allocated on first use
         self._meta_dev = None       # a spill's staged metadata (fixed address, see _stage_meta)
@@ -203,7 +205,8 @@ class KittyInferencePipeline:
         if not self._on_device:
             return torch.from_numpy(a)
         if self._stager is None:
-            self._stager = HostStager(self.device, 16 + 12 * self.num_slots)
+            # rows for a spill's metadata and for the page ids of most prompts
+            self._stager = HostStager(self.device, max(16 + 12 * self.num_slots, 4096))
         return self._stager(a, out) if out is not None else self._stager(a).view(a.shape)
 
     def _slots_tensor(self, slots: np.ndarray) -> torch.Tensor:
@@ -658,9 +661,11 @@ class KittyInferencePipeline:
                           seq_ids: Sequence[int]) -> None:
         """push_chunk for sequences that hold nothing yet at layer l (a new
         prompt), batched over the sequences: the same state as the
-        per-sequence path, from one copy per buffer kind, one key-page and one
-        value-page quantise launch for all of them (reading the pages in place
-        from the prompt tensors), and one counter write."""
+        per-sequence path.  On the device, a run of slots and prompts that
+        kernels can read in place take three steps (_push_prompt); otherwise
+        one copy per buffer kind, one key-page and one value-page quantise
+        launch for all of them (reading the pages in place from the prompt
+        tensors), and one counter write."""
         cfg = self.config
         S, G, R = cfg.sink_size, cfg.q_buffer_size, cfg.local_value_window
         B, H, T, D = keys.shape
@@ -670,6 +675,10 @@ class KittyInferencePipeline:
         v_full = n_full if R == 0 else max(0, (m - R) // G)  # of them, pages whose value half fills now
         rem, vrem = m - n_full * G, m - v_full * G
         phys = self._alloc_spill(l, slots, seq_ids, [n_full] * B) if n_full else []   # all or nothing
+        if (self._on_device and (H, D) == (cfg.num_kv_heads, cfg.head_dim) and values.shape == keys.shape and D % 8 == 0
+                and len(slots) == B <= 65535 and _is_run(slots) and plain_rows(keys, values)):
+            self._push_prompt(l, keys, values, slots, np.asarray(phys, np.int32), n_s, n_full, v_full)
+            return
         # one ascending run of slots (the usual case) is written through a
         # slice: plain strided copies instead of indexed scatters
         sl = slice(int(slots[0]), int(slots[0]) + B) if _is_run(slots) else self._slots_tensor(slots).long()
@@ -701,6 +710,55 @@ class KittyInferencePipeline:
         self._npv[slots, l] = v_full
         self._vlen[slots, l] = vrem
         self.lens[:, l, sl] = self._h2d(self._counts[:, slots, l])
+
+    def _push_prompt(self, l: int, keys: torch.Tensor, values: torch.Tensor, slots: np.ndarray, phys: np.ndarray,
+                     n_s: int, n_full: int, v_full: int) -> None:
+        """_push_chunk_fresh on the device for a run of slots: the page ids in one
+        staged copy, one quantise launch for the pages of keys and values
+        (two when more than 1,024 blocks would read values that stay FP16,
+        about what a launch costs), one kitty_store_prompt launch for the FP16
+        rows, the block table and the counters."""
+        cfg = self.config
+        G, n, maxp = cfg.q_buffer_size, self.num_slots, self.max_pages_per_seq
+        B, H, T, D = keys.shape
+        s0, st = int(slots[0]), slice(int(slots[0]), int(slots[0]) + B)
+        pages = None
+        if n_full:
+            both = v_full > 0 and (n_full - v_full) * B * H <= 1024
+            ids = np.empty((2 if v_full else 1, B, n_full), np.int32)
+            ids[0] = phys.reshape(B, n_full)
+            if v_full:
+                ids[1] = ids[0]
+                ids[1, :, v_full:] = -1            # value blocks past v_full write nothing
+            pages = self._h2d(ids.ravel())
+            blocks = lambda x, k: x[:, :, n_s:n_s + k * G].unflatten(2, (k, G)).transpose(1, 2)  # (B, k, H, G, D)
+            kpages = pages[:B * n_full]
+            QuantizePlan(self._store, blocks(keys, n_full), blocks(values, n_full) if both else None,
+                         self.boost_idx_uint8[l], kpages, cfg.sentinel,
+                         value_page_ids=pages[B * n_full:] if both else None).run()
+            if v_full and not both:
+                vpages = kpages.view(B, n_full)[:, :v_full].contiguous().view(-1)
+                quantize_into_pools(self._store, None, blocks(values, v_full), None, vpages, cfg.sentinel)
+        a = _hip.PromptArgs()
+        a.key, a.value = keys.data_ptr(), values.data_ptr()
+        a.key_s_seq, a.key_s_head, a.key_s_tok = keys.stride()[:3]
+        a.value_s_seq, a.value_s_head, a.value_s_tok = values.stride()[:3]
+        sk, sv, qk, vb = (t[s0, l] for t in (self._sink_k, self._sink_v, self._qbuf_k, self._vbuf))
+        layout = lambda t: _hip.SlotLayout(t.stride(0), t.stride(2), t.stride(3))
+        a.sink_k, a.sink_v, a.sink_layout = sk.data_ptr(), sv.data_ptr(), layout(self._sink_k)
+        a.key_buf, a.key_layout = qk.data_ptr(), layout(self._qbuf_k)
+        a.value_buf, a.value_layout = vb.data_ptr(), layout(self._vbuf)
+        a.counters = self.lens.data_ptr() + 4 * (l * n + s0)
+        a.counters_stride = cfg.num_layers * n
+        a.block_table, a.bt_stride = self._block_table.data_ptr() + 4 * (l * n + s0) * maxp, maxp
+        a.pages = pages.data_ptr() if pages is not None else None
+        a.batch, a.num_kv_heads, a.head_dim, a.tokens, a.page_tokens = B, H, D, T, G
+        a.n_sink, a.key_pages, a.value_pages = n_s, n_full, v_full
+        _hip.check(self._lib.kitty_store_prompt(ctypes.byref(a), _hip.stream_ptr(self.device)))
+        m = T - n_s
+        self._counts[:, st, l] = np.array([n_s, m - n_full * G, n_full, v_full, m - v_full * G])[:, None]
+        if n_full:
+            self._pages[st, l, :n_full] = ids[0]
 
     # ------------------------------------------------------------- query
     def get_attention_context(self, layer_id: int, seq_id: int = 0) -> dict:
@@ -759,12 +817,26 @@ class KittyInferencePipeline:
             return
         self._seq_of.pop(s, None)
         self._slots_of_ids.clear()
-        for c in (self._fill, self._qlen, self._npages, self._npv, self._vlen):
-            c[s] = 0
+        self._counts[:, s] = 0
         self._pages[s] = 0
+        if self._on_device:      # one launch for the buffers, the block table rows and the counters
+            regions = self._reset_regions.get(s)
+            if regions is None:
+                regions = self._reset_regions[s] = self._slot_regions(s)
+            _hip.check(self._lib.kitty_zero_regions(regions, len(regions), _hip.stream_ptr(self.device)))
+            return
         self.lens[:, :, s] = 0
         for t in (self._sink_k, self._sink_v, self._qbuf_k, self._vbuf, self._block_table.transpose(0, 1)):
             t[s].zero_()
+
+    def _slot_regions(self, s: int) -> ctypes.Array:
+        """kitty_zero_regions' list for slot s: what of the device state belongs to it."""
+        n, L, maxp = self.num_slots, self.config.num_layers, self.max_pages_per_seq
+        regions = [_hip.ZeroRegion(t[s].data_ptr(), 1, t[s].numel() * t.element_size(), 0)
+                   for t in (self._sink_k, self._sink_v, self._qbuf_k, self._vbuf)]
+        regions.append(_hip.ZeroRegion(self._block_table.data_ptr() + 4 * s * maxp, L, 4 * maxp, 4 * n * maxp))
+        regions.append(_hip.ZeroRegion(self.lens.data_ptr() + 4 * s, 5 * L, 4, 4 * n))
+        return (_hip.ZeroRegion * len(regions))(*regions)
 
     def stats(self) -> dict:
         return {
