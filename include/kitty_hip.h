@@ -248,9 +248,12 @@ typedef struct {
 
     /* element types (ABI version 3): the metadata pools, and q with the
      * sinks and tails.  out is fp16 either way, as the reference returns
-     * (kitty/kernels/attention.py:189). */
+     * (kitty/kernels/attention.py:189), unless out_dtype asks for bf16: the
+     * fp16 result converted once more, as a module whose queries are bf16
+     * returns it (kitty/attention.py:151; ABI version 7). */
     int32_t meta_dtype; /* KITTY_DTYPE_F16 or KITTY_DTYPE_BF16 */
     int32_t act_dtype;  /* KITTY_DTYPE_F16 or KITTY_DTYPE_BF16 */
+    int32_t out_dtype;  /* KITTY_DTYPE_F16 or KITTY_DTYPE_BF16 */
 } kitty_decode_args;
 
 int kitty_decode_workspace_size(const kitty_decode_args *args, size_t *bytes);
@@ -333,6 +336,12 @@ typedef struct {
 } kitty_append_args;
 
 int kitty_append_tokens(const kitty_append_args *args, kitty_stream_t stream);
+
+/* One decode step of a batch whose buffers do not fill with this token:
+ * kitty_append_tokens followed by kitty_paged_decode on the same stream, one
+ * call (kitty/attention.py:74-151, ABI version 7).  The decode's arguments are
+ * checked before anything is launched. */
+int kitty_decode_step(const kitty_append_args *append, const kitty_decode_args *decode, kitty_stream_t stream);
 
 /* ------------------------------------------------- prompt attention
  * Replaces the scaled_dot_product_attention call of the T > 1 branch of

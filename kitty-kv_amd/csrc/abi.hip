@@ -122,6 +122,8 @@ static int build_params(const kitty_decode_args *args, DecodeParams &p)
     if ((a.meta_dtype != KITTY_DTYPE_F16 && a.meta_dtype != KITTY_DTYPE_BF16) ||
         (a.act_dtype != KITTY_DTYPE_F16 && a.act_dtype != KITTY_DTYPE_BF16))
         return fail(KITTY_E_INVALID, "meta_dtype and act_dtype must be KITTY_DTYPE_F16 or KITTY_DTYPE_BF16");
+    if (a.out_dtype != KITTY_DTYPE_F16 && a.out_dtype != KITTY_DTYPE_BF16)
+        return fail(KITTY_E_INVALID, "out_dtype must be KITTY_DTYPE_F16 or KITTY_DTYPE_BF16");
     p = DecodeParams{};
     p.q = a.q;
     p.q_s_seq = a.q_s_seq;
@@ -159,6 +161,7 @@ static int build_params(const kitty_decode_args *args, DecodeParams &p)
     p.flags = a.flags;
     p.meta_bf16 = a.meta_dtype == KITTY_DTYPE_BF16;
     p.act_bf16 = a.act_dtype == KITTY_DTYPE_BF16;
+    p.out_bf16 = a.out_dtype == KITTY_DTYPE_BF16;
     p.sm_scale = a.sm_scale;
     p.gq_stride = a.num_q_heads / a.num_kv_heads;
     p.sub_groups = (p.gq_stride + 15) / 16;
@@ -325,12 +328,10 @@ extern "C" int kitty_paged_decode_merge(const kitty_decode_args *args, kitty_str
     return launch_merge(p, (hipStream_t)stream);
 }
 
-extern "C" int kitty_paged_decode(const kitty_decode_args *args, kitty_stream_t stream)
+// The launches of a prepared decode, one split + merge per sub-group.
+static int launch_decode(DecodeParams &p, const kitty_decode_args *args, kitty_stream_t stream)
 {
-    DecodeParams p;
-    int rc = prepare(args, p);
-    if (rc || p.B == 0)
-        return rc;
+    int rc = KITTY_OK;
     for (int s = 0; s < p.sub_groups; ++s) {
         if (s > 0) {
             sub_group(p, *args, s);
@@ -344,6 +345,23 @@ extern "C" int kitty_paged_decode(const kitty_decode_args *args, kitty_stream_t 
             return rc;
     }
     return KITTY_OK;
+}
+
+extern "C" int kitty_paged_decode(const kitty_decode_args *args, kitty_stream_t stream)
+{
+    DecodeParams p;
+    const int rc = prepare(args, p);
+    return rc || p.B == 0 ? rc : launch_decode(p, args, stream);
+}
+
+extern "C" int kitty_decode_step(const kitty_append_args *append, const kitty_decode_args *decode, kitty_stream_t stream)
+{
+    DecodeParams p;
+    int rc = prepare(decode, p);
+    if (rc)
+        return rc;
+    rc = kitty_append_tokens(append, stream);
+    return rc || p.B == 0 ? rc : launch_decode(p, decode, stream);
 }
 
 // ------------------------------------------------------------ no-alloc

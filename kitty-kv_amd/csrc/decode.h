@@ -43,6 +43,7 @@ struct DecodeParams {
     int flags;
     int meta_bf16; // metadata pools hold bf16 (else fp16)
     int act_bf16;  // q, sinks and tails hold bf16 (else fp16)
+    int out_bf16;  // out is written as bf16(fp16(x)) (else fp16)
     float sm_scale;
     // Unit-balanced plan of the MFMA kernel (balanced = 1): the grid has
     // page_waves waves (plan_waves says how many work); fp16_weight = units

@@ -308,6 +308,13 @@ __device__ __forceinline__ float wave_sum(float v)
     return v;
 }
 
+// An output value's bits: fp16, or the fp16 value converted to bf16.
+__device__ __forceinline__ uint16_t out_bits(const DecodeParams &p, float v)
+{
+    const uint16_t h = f2h(v);
+    return p.out_bf16 ? f2bf(h2f(h)) : h;
+}
+
 // Merge of NS <= N partials (N <= 128; rows row0 + s * rstep) in one round
 // trip: lane l holds (m, l) of partials l and l + 64, every lane loads the N
 // O rows of its channel pair (rows past NS repeat the last, with weight 0).
@@ -345,10 +352,10 @@ __device__ __forceinline__ void merge_one_pass(const DecodeParams &p, int64_t ro
     if (d < p.D) {
         const float x = nan ? __builtin_nanf("") : ax * inv, y = nan ? __builtin_nanf("") : ay * inv;
         if (((uintptr_t)o & 3) == 0) {
-            *(uint32_t *)(o + d) = (uint32_t)f2h(x) | ((uint32_t)f2h(y) << 16);
+            *(uint32_t *)(o + d) = (uint32_t)out_bits(p, x) | ((uint32_t)out_bits(p, y) << 16);
         } else {
-            o[d] = f2h(x);
-            o[d + 1] = f2h(y);
+            o[d] = out_bits(p, x);
+            o[d + 1] = out_bits(p, y);
         }
     }
 }
@@ -414,7 +421,7 @@ __device__ __forceinline__ void merge_quads(const DecodeParams &p, int64_t row0,
     uint16_t h[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-        h[e] = f2h(nan ? __builtin_nanf("") : acc[e] * inv);
+        h[e] = out_bits(p, nan ? __builtin_nanf("") : acc[e] * inv);
     uint16_t *dst = o + 8 * c;
     if (((uintptr_t)dst & 15) == 0) {
         *(u32x4 *)dst = u32x4{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
@@ -524,10 +531,10 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(DecodeParams p)
         if (d < p.D) {
             const float x = nan ? __builtin_nanf("") : ax * inv, y = nan ? __builtin_nanf("") : ay * inv;
             if (((uintptr_t)o & 3) == 0) {
-                *(uint32_t *)(o + d) = (uint32_t)f2h(x) | ((uint32_t)f2h(y) << 16);
+                *(uint32_t *)(o + d) = (uint32_t)out_bits(p, x) | ((uint32_t)out_bits(p, y) << 16);
             } else {
-                o[d] = f2h(x);
-                o[d + 1] = f2h(y);
+                o[d] = out_bits(p, x);
+                o[d + 1] = out_bits(p, y);
             }
         }
     }

@@ -95,7 +95,7 @@ class DecodeArgs(ctypes.Structure):
         ("flags", _i32), ("sm_scale", ctypes.c_float),
         ("workspace", _vp), ("workspace_bytes", ctypes.c_size_t),
         ("num_pages_v", _vp), ("tail_len_v", _vp), ("tail_v_capacity", _i32),
-        ("meta_dtype", _i32), ("act_dtype", _i32),
+        ("meta_dtype", _i32), ("act_dtype", _i32), ("out_dtype", _i32),
     ]
 
 
@@ -156,7 +156,7 @@ EXPORTED_SYMBOLS = (
     "kitty_paged_decode_merge", "kitty_paged_decode_noalloc", "kitty_append_tokens", "kitty_channel_abs_sum",
     "kitty_channel_abs_sum_workspace_size", "kitty_channel_abs_sum_deferred_size", "kitty_channel_abs_sum_deferred",
     "kitty_channel_abs_sum_flush", "kitty_store_i32", "kitty_prefill_attention",
-    "kitty_store_prompt", "kitty_zero_regions",
+    "kitty_store_prompt", "kitty_zero_regions", "kitty_decode_step",
 )
 
 _lib: Optional[ctypes.CDLL] = None
@@ -195,6 +195,7 @@ def load() -> ctypes.CDLL:
     L.kitty_channel_abs_sum_deferred.argtypes = L.kitty_channel_abs_sum.argtypes
     L.kitty_channel_abs_sum_flush.argtypes = [_vp, _i32, _i32, _vp, _vp]
     L.kitty_store_i32.argtypes = [_vp, _vp, _i32, _vp]
+    L.kitty_decode_step.argtypes = [ctypes.POINTER(AppendArgs), ctypes.POINTER(DecodeArgs), _vp]
     L.kitty_store_prompt.argtypes = [ctypes.POINTER(PromptArgs), _vp]
     L.kitty_zero_regions.argtypes = [ctypes.POINTER(ZeroRegion), _i32, _vp]
     L.kitty_prefill_attention.argtypes = [ctypes.POINTER(PrefillArgs), _vp]

@@ -371,6 +371,7 @@ class DecodePlan:
             workspace = torch.empty(max(need.value, 16), dtype=torch.uint8, device=dev)
         a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
         self.args = a
+        self._step: Optional[_hip.DecodeArgs] = None
         self.out = out
         self.device = dev
         self._sig = ((q.device, q.dtype, q.shape, q.stride()), (out.device, out.dtype, out.shape, out.stride()))
@@ -395,6 +396,28 @@ class DecodePlan:
         finally:
             self.args.q, self.args.out = self._keep[0].data_ptr(), self.out.data_ptr()
         return out
+
+    def step_args(self, q: torch.Tensor, out: torch.Tensor) -> _hip.DecodeArgs:
+        """The plan's arguments for a contiguous (B, Hq, 1, D) query of the
+        plan's dtype on its device and an output like it (fp16, or bf16 from
+        the fp16 result), in one structure that the next call of step_args
+        overwrites."""
+        B, Hq, D = self._sig[0][2]
+        _need(tuple(q.shape) == (B, Hq, 1, D) and (q.device, q.dtype) == self._sig[0][:2] and q.shape == out.shape
+              and out.dtype == q.dtype, "q and out must match the plan")
+        a = self._step
+        if a is None:
+            a = self._step = _hip.DecodeArgs()
+            ctypes.memmove(ctypes.byref(a), ctypes.byref(self.args), ctypes.sizeof(a))
+            a.q_s_seq = a.out_s_seq = Hq * D
+            a.q_s_head = a.out_s_head = D
+            a.out_dtype = _hip.dtype_code(out, "out")
+        a.q, a.out = q.data_ptr(), out.data_ptr()
+        return a
+
+    def run_args(self, args: _hip.DecodeArgs) -> None:
+        """The decode of step_args on the current stream."""
+        _hip.check(self._L.kitty_paged_decode(ctypes.byref(args), _hip.stream_ptr(self.device)))
 
     def run_splits(self) -> None:
         _hip.check(self._L.kitty_paged_decode_splits(ctypes.byref(self.args), _hip.stream_ptr(self.device)))

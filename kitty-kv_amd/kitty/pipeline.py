@@ -112,6 +112,7 @@ class KittyInferencePipeline:
         self._slots_dev: Dict[Tuple[int, ...], torch.Tensor] = {}
         # slot arrays of batches of sequence ids seen before (cleared when a slot is freed)
         self._slots_of_ids: Dict[Tuple[int, ...], np.ndarray] = {}
+        self._slot_epoch = 0        # advances whenever a slot is freed: slots cached by id are stale then
         # append arguments per (layer, slots): everything but the token pointers
         self._append_args: Dict[Tuple[int, Tuple[int, ...]], Tuple[_hip.AppendArgs, torch.Tensor]] = {}
         # per slot: the device regions reset_sequence zeroes
@@ -226,6 +227,13 @@ class KittyInferencePipeline:
 
     def push_tokens(self, layer_id: int, keys: torch.Tensor, values: torch.Tensor, seq_ids: Sequence[int]) -> None:
         """One token for each of B sequences: keys / values (B, num_kv_heads, head_dim)."""
+        self._push(layer_id, keys, values, seq_ids, None)
+
+    def _push(self, layer_id: int, keys: torch.Tensor, values: torch.Tensor, seq_ids: Sequence[int],
+              decode: Optional[_hip.DecodeArgs]) -> bool:
+        """push_tokens; with the arguments of the decode that follows, a token
+        that fills no buffer is appended and decoded by one kitty_decode_step
+        call.  True when it was (a spill comes between the two otherwise)."""
         cfg = self.config
         S, G = cfg.sink_size, cfg.q_buffer_size
         ids = tuple(seq_ids)
@@ -253,7 +261,11 @@ class KittyInferencePipeline:
                 if pno + 1 > self.max_pages_per_seq:
                     raise RuntimeError(f"sequence {ids[0]} exceeds max_seq_len={cfg.max_seq_len}")
                 phys = self.layout.allocate_run(ids[0], l, pno, 1)
-            append(l, keys, values, slots)
+            if decode is not None and not (kf or vf):
+                self._append_device(l, keys, values, slots, decode)
+            else:
+                decode = None
+                append(l, keys, values, slots)
             if in_sink:
                 self._fill[s, l] += 1
             else:
@@ -264,7 +276,17 @@ class KittyInferencePipeline:
                     self._spill_one(l, s, kf, vf, phys)
                 else:
                     self._spill(l, slots if kf else slots[:0], phys, slots if vf else slots[:0])
-            return
+            return decode is not None
+        if decode is not None:
+            # the usual step of a batch: every sequence past its sinks, no
+            # buffer that this token fills
+            counts = self._counts[:, slots, l]
+            if (counts[_FILL].min() >= S and counts[_QLEN].max() + 1 < G
+                    and counts[_VLEN].max() + 1 < self.value_capacity):
+                self._append_device(l, keys, values, slots, decode)
+                self._qlen[slots, l] = counts[_QLEN] + 1
+                self._vlen[slots, l] = counts[_VLEN] + 1
+                return True
         fill = self._fill[slots, l]
         in_sink = fill < S
         rows = np.nonzero(~in_sink)[0]
@@ -279,9 +301,12 @@ class KittyInferencePipeline:
         self._vlen[slots[rows], l] += 1
         if len(kfull) or len(vfull):
             self._spill(l, slots[kfull], phys, slots[vfull])
+        return False
 
-    def _append_device(self, l: int, keys: torch.Tensor, values: torch.Tensor, slots: np.ndarray) -> None:
-        """kitty_append_tokens: every sequence's token into its buffers, one launch."""
+    def _append_device(self, l: int, keys: torch.Tensor, values: torch.Tensor, slots: np.ndarray,
+                       decode: Optional[_hip.DecodeArgs] = None) -> None:
+        """kitty_append_tokens: every sequence's token into its buffers, one
+        launch; with `decode`, kitty_decode_step: the decode behind it."""
         keys = keys if keys.stride(-1) == 1 else keys.contiguous()
         values = values if values.stride(-1) == 1 else values.contiguous()
         ck = (l, tuple(slots.tolist()))
@@ -295,7 +320,11 @@ class KittyInferencePipeline:
         a.key, a.value = keys.data_ptr(), values.data_ptr()
         a.key_s_seq, a.key_s_head = keys.stride(0), keys.stride(1)
         a.value_s_seq, a.value_s_head = values.stride(0), values.stride(1)
-        _hip.check(self._lib.kitty_append_tokens(ctypes.byref(a), _hip.stream_ptr(self.device)))
+        stream = _hip.stream_ptr(self.device)
+        if decode is None:
+            _hip.check(self._lib.kitty_append_tokens(ctypes.byref(a), stream))
+        else:
+            _hip.check(self._lib.kitty_decode_step(ctypes.byref(a), ctypes.byref(decode), stream))
 
     def _append_setup(self, l: int, slots: np.ndarray, H: int, D: int) -> Tuple[_hip.AppendArgs, torch.Tensor]:
         """kitty_append_tokens arguments of layer l for these slots, bar the
@@ -817,6 +846,7 @@ class KittyInferencePipeline:
             return
         self._seq_of.pop(s, None)
         self._slots_of_ids.clear()
+        self._slot_epoch += 1
         self._counts[:, s] = 0
         self._pages[s] = 0
         if self._on_device:      # one launch for the buffers, the block table rows and the counters
