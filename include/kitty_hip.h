@@ -465,6 +465,32 @@ int kitty_channel_abs_sum_deferred(const uint16_t *key, int64_t s_b, int64_t s_t
 int kitty_channel_abs_sum_flush(void *slots, int32_t num_kv_heads, int32_t head_dim, float *out,
                                 kitty_stream_t stream);
 
+/* The deferred call on a slot buffer whose contents do not count (the first
+ * batch, or the first after its sums were read): every slot is written, so the buffer
+ * needs no zeroing (ABI version 7).  Shapes without slots return
+ * KITTY_E_UNSUPPORTED. */
+int kitty_channel_abs_sum_first(const uint16_t *key, int64_t s_b, int64_t s_t, int64_t s_h, int32_t batch,
+                                int32_t tokens, int32_t num_kv_heads, int32_t head_dim, int32_t key_dtype,
+                                void *slots, size_t slots_bytes, kitty_stream_t stream);
+
+/* Sums, scores and ranks of n layers in one launch per KITTY_SCORE_LAYERS of
+ * them (KittySensitivityProfiler.compute, kitty/sensitivity.py:164-207; ABI
+ * version 7): for layer i, sum = (add_to_sum ? sum_abs : 0) + the slots' sums
+ * (slots NULL: none) is stored to sum_abs, scores[i][h][d] = sum * (1 / tokens),
+ * and boost_idx[i][h][d] is d's rank in descending score order (NaN first, equal
+ * scores by channel) where below d_boost, else the sentinel.  The slots' contents
+ * no longer count afterwards.  head_dim at most 512. */
+#define KITTY_SCORE_LAYERS 64
+typedef struct {
+    const float *slots;
+    float *sum_abs;
+    float tokens;
+    int32_t add_to_sum;
+} kitty_score_layer;
+
+int kitty_channel_scores(const kitty_score_layer *layers, int32_t n, int32_t num_kv_heads, int32_t head_dim,
+                         int32_t d_boost, int32_t sentinel, float *scores, uint8_t *boost_idx, kitty_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -67,9 +67,11 @@ __device__ __forceinline__ float abs_h(unsigned w, bool hi, bool bf16)
 }
 
 // Chunk c's D sums go to ws[(h * D + d) * slots + c]: written (slots =
-// S.chunks, the two-pass call) or added to the slot's running sum (slots =
+// S.chunks, the two-pass call), added to the slot's running sum (slots =
 // kMaxChunks, the deferred call; one workgroup per slot and call, so the
-// order of the additions is that of the calls).
+// order of the additions is that of the calls), or written with the slots no
+// chunk has set to zero (kMaxChunks, the first call on a buffer: no fill of
+// 1 MB per layer before it).
 __global__ __launch_bounds__(kSumThreads) void abs_sum_chunks_kernel(const uint16_t *key, int64_t s_b, int64_t s_t,
                                                                      int64_t s_h, AbsSumShape S, bool bf16,
                                                                      float *ws, int slots, bool add)
@@ -124,6 +126,9 @@ __global__ __launch_bounds__(kSumThreads) void abs_sum_chunks_kernel(const uint1
         if (add)
             sum += d == tid ? prev : *slot;  // d >= 256 (head_dim above 256): loaded here
         *slot = sum;
+        if (!add)
+            for (int z = c + S.chunks; z < slots; z += S.chunks)
+                slot[z - c] = 0.0f;
     }
 }
 
@@ -183,6 +188,66 @@ __global__ __launch_bounds__(1024) void abs_sum_rows_kernel(const uint16_t *key,
         for (int i = 0; i < 16; ++i)
             s += red[i][lane];
         out[h * D + d] += s;
+    }
+}
+
+// Scores and ranks (kitty_channel_scores): one 1024-thread workgroup per (layer,
+// head).  Each wave sums the slots of every 16th channel in the order of
+// abs_sum_finish_kernel, four channels' loads in flight; the ranks are counted by
+// comparing every channel with every other in LDS.
+constexpr int kScoreThreads = 1024;
+constexpr int kScoreChannels = 512;
+
+struct ScoreArgs {
+    kitty_score_layer layer[KITTY_SCORE_LAYERS];
+};
+static_assert(sizeof(ScoreArgs) <= 3072, "kernel arguments above 4 KB");
+
+// a ranks before b: greater, NaN above every number
+__device__ __forceinline__ bool ranks_before(float a, float b) { return a > b || (a != a && b == b); }
+
+__global__ __launch_bounds__(kScoreThreads) void channel_scores_kernel(ScoreArgs a, int H, int D, int d_boost, int sentinel,
+                                                                       float *scores, uint8_t *boost_idx)
+{
+    __shared__ float sc[kScoreChannels];
+    const int h = blockIdx.x, i = blockIdx.y;
+    const kitty_score_layer L = a.layer[i];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const float inv = 1.0f / L.tokens;
+    for (int d0 = wave * 4; d0 < D; d0 += 4 * (kScoreThreads / 64)) {
+        float v[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                v[u][c] = L.slots ? L.slots[((int64_t)h * D + min(d0 + u, D - 1)) * kMaxChunks + 64 * c + lane] : 0.0f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                sum += v[u][c];
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1)
+                sum += __shfl_xor(sum, off);
+            const int d = d0 + u;
+            if (lane == 0 && d < D) {
+                float *out = L.sum_abs + (int64_t)h * D + d;
+                const float total = L.add_to_sum ? *out + sum : sum;
+                *out = total;
+                sc[d] = total * inv;
+            }
+        }
+    }
+    __syncthreads();
+    for (int d = threadIdx.x; d < D; d += kScoreThreads) {
+        const float mine = sc[d];
+        int rank = 0;
+        for (int e = 0; e < D; ++e)
+            rank += ranks_before(sc[e], mine) || (e < d && !ranks_before(mine, sc[e])) ? 1 : 0;
+        const int64_t o = ((int64_t)i * H + h) * D + d;
+        scores[o] = mine;
+        boost_idx[o] = (uint8_t)(rank < d_boost ? rank : sentinel);
     }
 }
 
@@ -304,4 +369,60 @@ extern "C" int kitty_channel_abs_sum_flush(void *slots, int32_t num_kv_heads, in
     hipLaunchKernelGGL(abs_sum_finish_kernel, dim3((num_kv_heads * head_dim + 3) / 4), dim3(256), 0,
                        (hipStream_t)stream, (float *)slots, S, out, kMaxChunks, true);
     return check_launch("abs_sum_finish_kernel");
+}
+
+extern "C" int kitty_channel_abs_sum_first(const uint16_t *key, int64_t s_b, int64_t s_t, int64_t s_h, int32_t batch,
+                                           int32_t tokens, int32_t num_kv_heads, int32_t head_dim, int32_t key_dtype,
+                                           void *slots, size_t slots_bytes, kitty_stream_t stream)
+{
+    if (batch <= 0 || tokens <= 0 || num_kv_heads <= 0 || head_dim <= 0)
+        return fail(KITTY_E_INVALID, "bad shape");
+    if (key_dtype != KITTY_DTYPE_F16 && key_dtype != KITTY_DTYPE_BF16)
+        return fail(KITTY_E_INVALID, "key_dtype must be KITTY_DTYPE_F16 or KITTY_DTYPE_BF16");
+    if (!key || !slots)
+        return fail(KITTY_E_INVALID, "NULL key or slots");
+    if (!split_ok(key, s_b, s_t, s_h, head_dim))
+        return fail(KITTY_E_UNSUPPORTED, "no slots for this shape: use kitty_channel_abs_sum_deferred");
+    const size_t need = (size_t)num_kv_heads * head_dim * kMaxChunks * sizeof(float);
+    if (slots_bytes < need)
+        return fail(KITTY_E_INVALID, "slot buffer too small: need " + std::to_string(need) + " bytes");
+    if ((uintptr_t)slots & 15)
+        return fail(KITTY_E_INVALID, "slot buffer must be 16-byte aligned");
+    const AbsSumShape S = abs_sum_shape(batch, tokens, num_kv_heads, head_dim);
+    hipLaunchKernelGGL(abs_sum_chunks_kernel, dim3(S.chunks, num_kv_heads), dim3(kSumThreads), 0, (hipStream_t)stream, key,
+                       s_b, s_t, s_h, S, key_dtype == KITTY_DTYPE_BF16, (float *)slots, kMaxChunks, false);
+    return check_launch("abs_sum_chunks_kernel");
+}
+
+extern "C" int kitty_channel_scores(const kitty_score_layer *layers, int32_t n, int32_t num_kv_heads, int32_t head_dim,
+                                    int32_t d_boost, int32_t sentinel, float *scores, uint8_t *boost_idx,
+                                    kitty_stream_t stream)
+{
+    if (n < 0 || num_kv_heads <= 0 || head_dim <= 0 || d_boost < 0 || sentinel < 0 || sentinel > 255 || d_boost > 256)
+        return fail(KITTY_E_INVALID, "bad shape, d_boost or sentinel");
+    if (head_dim > kScoreChannels)
+        return fail(KITTY_E_UNSUPPORTED, "kitty_channel_scores: head_dim above 512");
+    if (n == 0)
+        return KITTY_OK;
+    if (!layers || !scores || !boost_idx)
+        return fail(KITTY_E_INVALID, "NULL layers, scores or boost_idx");
+    for (int32_t i = 0; i < n; ++i) {
+        if (!layers[i].sum_abs || !(layers[i].tokens > 0.0f))
+            return fail(KITTY_E_INVALID, "kitty_channel_scores: a layer without sums or tokens");
+        if (layers[i].slots && !abs_sum_split_shape(head_dim))
+            return fail(KITTY_E_INVALID, "kitty_channel_scores: this head_dim has no slots");
+    }
+    for (int32_t i0 = 0; i0 < n; i0 += KITTY_SCORE_LAYERS) {
+        ScoreArgs a{};
+        const int m = n - i0 < KITTY_SCORE_LAYERS ? n - i0 : KITTY_SCORE_LAYERS;
+        for (int i = 0; i < m; ++i)
+            a.layer[i] = layers[i0 + i];
+        const int64_t o = (int64_t)i0 * num_kv_heads * head_dim;
+        hipLaunchKernelGGL(channel_scores_kernel, dim3(num_kv_heads, m), dim3(kScoreThreads), 0, (hipStream_t)stream, a,
+                           num_kv_heads, head_dim, d_boost, sentinel, scores + o, boost_idx + o);
+        const int rc = check_launch("channel_scores_kernel");
+        if (rc != KITTY_OK)
+            return rc;
+    }
+    return KITTY_OK;
 }

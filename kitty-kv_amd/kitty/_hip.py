@@ -118,6 +118,10 @@ class AppendArgs(ctypes.Structure):
     ]
 
 
+class ScoreLayer(ctypes.Structure):
+    _fields_ = [("slots", _vp), ("sum_abs", _vp), ("tokens", ctypes.c_float), ("add_to_sum", _i32)]
+
+
 class PromptArgs(ctypes.Structure):
     """kitty_prompt_args: the FP16 rows, table entries and counters of new prompts."""
     _fields_ = [
@@ -156,7 +160,8 @@ EXPORTED_SYMBOLS = (
     "kitty_paged_decode_merge", "kitty_paged_decode_noalloc", "kitty_append_tokens", "kitty_channel_abs_sum",
     "kitty_channel_abs_sum_workspace_size", "kitty_channel_abs_sum_deferred_size", "kitty_channel_abs_sum_deferred",
     "kitty_channel_abs_sum_flush", "kitty_store_i32", "kitty_prefill_attention",
-    "kitty_store_prompt", "kitty_zero_regions", "kitty_decode_step",
+    "kitty_store_prompt", "kitty_zero_regions", "kitty_decode_step", "kitty_channel_abs_sum_first",
+    "kitty_channel_scores",
 )
 
 _lib: Optional[ctypes.CDLL] = None
@@ -195,6 +200,9 @@ def load() -> ctypes.CDLL:
     L.kitty_channel_abs_sum_deferred.argtypes = L.kitty_channel_abs_sum.argtypes
     L.kitty_channel_abs_sum_flush.argtypes = [_vp, _i32, _i32, _vp, _vp]
     L.kitty_store_i32.argtypes = [_vp, _vp, _i32, _vp]
+    L.kitty_channel_abs_sum_first.argtypes = [_vp, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t,
+                                              _vp]
+    L.kitty_channel_scores.argtypes = [ctypes.POINTER(ScoreLayer), _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp]
     L.kitty_decode_step.argtypes = [ctypes.POINTER(AppendArgs), ctypes.POINTER(DecodeArgs), _vp]
     L.kitty_store_prompt.argtypes = [ctypes.POINTER(PromptArgs), _vp]
     L.kitty_zero_regions.argtypes = [ctypes.POINTER(ZeroRegion), _i32, _vp]

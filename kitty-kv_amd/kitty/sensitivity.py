@@ -37,13 +37,24 @@ class _ChannelAccumulator:
     def __init__(self, num_kv_heads: int, head_dim: int, device) -> None:
         self.num_kv_heads = num_kv_heads
         self.head_dim = head_dim
-        self._sum_abs = torch.zeros(num_kv_heads, head_dim, dtype=torch.float32, device=device)
+        self._sum_device = torch.device(device)
+        self._sum: Optional[torch.Tensor] = None      # Σ|k| of what was read so far, made on first use
         self.token_count = 0
-        # per-chunk running sums of the deferred kernel (zero between flushes),
-        # added into _sum_abs when sum_abs is read: one pass over the keys per
-        # update, the finishing pass once per read
+        # per-chunk running sums of the deferred kernel, added into the sums
+        # when sum_abs is read: one pass over the keys per update, the
+        # finishing pass once per read.  Their contents count while _pending.
         self._slots: Optional[torch.Tensor] = None
         self._pending = False
+
+    @property
+    def _sum_abs(self) -> torch.Tensor:
+        if self._sum is None:
+            self._sum = torch.zeros(self.num_kv_heads, self.head_dim, dtype=torch.float32, device=self._sum_device)
+        return self._sum
+
+    @_sum_abs.setter
+    def _sum_abs(self, t: torch.Tensor) -> None:
+        self._sum, self._sum_device = t, t.device
 
     @property
     def sum_abs(self) -> torch.Tensor:
@@ -67,7 +78,9 @@ class _ChannelAccumulator:
             self.token_count += B * T
             return
         dev = _hip.require_device(key)
-        if self._sum_abs.device != dev:
+        if self._sum is None and self._sum_device.type == "cuda" and self._sum_device.index is None:
+            self._sum_device = dev
+        if self._sum_device != dev:
             self._sum_abs = self.sum_abs.to(dev)      # pending slots flushed on the old device first
             self._slots = None
         if key.dtype not in (torch.float16, torch.bfloat16):
@@ -78,13 +91,24 @@ class _ChannelAccumulator:
         if self._slots is None:
             need = ctypes.c_size_t(0)
             _hip.check(L.kitty_channel_abs_sum_deferred_size(H, D, ctypes.byref(need)))
-            self._slots = torch.zeros(max(need.value, 16), dtype=torch.uint8, device=dev)
+            self._slots = torch.empty(max(need.value, 16), dtype=torch.uint8, device=dev)
             self._slots_bytes = need.value
+        # slots exist for rows of 16 bytes: other keys add into the sums at once
+        rows16 = (self._slots_bytes > 0 and key.data_ptr() % 16 == 0
+                  and not any(s % 8 for s in key.stride()[:3]))
+        if B * T == 0:
+            return
+        if rows16 and not self._pending:
+            _hip.check(L.kitty_channel_abs_sum_first(
+                key.data_ptr(), key.stride(0), key.stride(2), key.stride(1), B, T, H, D, _hip.dtype_code(key, "key"),
+                self._slots.data_ptr(), self._slots_bytes, _hip.stream_ptr(dev)))
+            self._pending = True
+            self.token_count += B * T
+            return
         _hip.check(L.kitty_channel_abs_sum_deferred(
             key.data_ptr(), key.stride(0), key.stride(2), key.stride(1), B, T, H, D, _hip.dtype_code(key, "key"),
-            self._sum_abs.data_ptr(), self._slots.data_ptr() if self._slots_bytes else None, self._slots_bytes,
+            self._sum_abs.data_ptr(), self._slots.data_ptr() if rows16 else None, self._slots_bytes,
             _hip.stream_ptr(dev)))
-        self._pending = self._slots_bytes > 0
         self.token_count += B * T
 
     def scores(self) -> torch.Tensor:
@@ -178,11 +202,47 @@ class KittySensitivityProfiler:
         if not self._accumulators:
             raise RuntimeError("No accumulators found.  Did you call register_hooks() and "
                                "forward the model over the calibration data?")
+        if self._compute_on_device():
+            return
         scores = torch.zeros(cfg.num_layers, cfg.num_kv_heads, cfg.head_dim, dtype=torch.float32)
         for layer_idx, acc in self._accumulators.items():
             scores[layer_idx] = acc.scores().cpu()
         self.scores_ = scores
         self.boost_masks_, self.boost_idx_uint8_ = rank_channels(scores, cfg.d_boost, cfg.sentinel)
+
+    def _compute_on_device(self) -> bool:
+        """compute() for accumulators of every layer on one ROCm device: sums,
+        scores and ranks by kitty_channel_scores, one copy to the host."""
+        cfg = self.config
+        H, D, n = cfg.num_kv_heads, cfg.head_dim, cfg.num_layers
+        accs = [self._accumulators.get(l) for l in range(n)]
+        if len(self._accumulators) != n or None in accs or D > 512 or cfg.d_boost > min(D, 255):
+            return False
+        dev = accs[0]._sum_device
+        if dev.type != "cuda" or dev.index is None:
+            return False
+        for acc in accs:
+            if acc._sum_device != dev or acc.token_count == 0 or (acc.num_kv_heads, acc.head_dim) != (H, D):
+                return False
+        layers = (_hip.ScoreLayer * n)()
+        fresh = [l for l, acc in enumerate(accs) if acc._sum is None]
+        sums = torch.empty(len(fresh), H, D, dtype=torch.float32, device=dev)
+        for l, acc in enumerate(accs):
+            old = acc._sum is not None
+            if not old:
+                acc._sum_abs = sums[fresh.index(l)]
+            layers[l] = _hip.ScoreLayer(acc._slots.data_ptr() if acc._pending else None, acc._sum.data_ptr(),
+                                        float(acc.token_count), int(old))
+        both = torch.empty(5 * n * H * D, dtype=torch.uint8, device=dev)     # scores (fp32), then ranks
+        _hip.check(_hip.load().kitty_channel_scores(layers, n, H, D, cfg.d_boost, cfg.sentinel, both.data_ptr(),
+                                                    both.data_ptr() + 4 * n * H * D, _hip.stream_ptr(dev)))
+        for acc in accs:
+            acc._pending = False
+        host = both.cpu()
+        self.scores_ = host[:4 * n * H * D].view(torch.float32).view(n, H, D).clone()
+        self.boost_idx_uint8_ = host[4 * n * H * D:].view(n, H, D).clone()
+        self.boost_masks_ = self.boost_idx_uint8_ < cfg.d_boost if cfg.d_boost > 0 else torch.zeros(n, H, D, dtype=torch.bool)
+        return True
 
     # ------------------------------------------------------------------- I/O
     def save(self, directory) -> None:
