@@ -254,6 +254,11 @@ typedef struct {
     int32_t meta_dtype; /* KITTY_DTYPE_F16 or KITTY_DTYPE_BF16 */
     int32_t act_dtype;  /* KITTY_DTYPE_F16 or KITTY_DTYPE_BF16 */
     int32_t out_dtype;  /* KITTY_DTYPE_F16 or KITTY_DTYPE_BF16 */
+
+    /* What the caller knows of the largest num_pages[b] (ABI version 7); 0:
+     * max_pages.  It only chooses between kernels, whose results are the same
+     * but for rounding. */
+    int32_t plan_pages;
 } kitty_decode_args;
 
 int kitty_decode_workspace_size(const kitty_decode_args *args, size_t *bytes);
@@ -340,8 +345,12 @@ int kitty_append_tokens(const kitty_append_args *args, kitty_stream_t stream);
 /* One decode step of a batch whose buffers do not fill with this token:
  * kitty_append_tokens followed by kitty_paged_decode on the same stream, one
  * call (kitty/attention.py:74-151, ABI version 7).  The decode's arguments are
- * checked before anything is launched. */
-int kitty_decode_step(const kitty_append_args *append, const kitty_decode_args *decode, kitty_stream_t stream);
+ * checked before anything is launched.  With tickets (device, an int32 per slot
+ * of the append, all 0; each call leaves them 0) a batch of few pairs and pages
+ * takes one launch, for which the decode's buffers and lengths have to be those
+ * the append writes (decode->sink_len[b] == append->sink_fill[slots[b]] and so on). */
+int kitty_decode_step(const kitty_append_args *append, const kitty_decode_args *decode, int32_t *tickets,
+                      kitty_stream_t stream);
 
 /* ------------------------------------------------- prompt attention
  * Replaces the scaled_dot_product_attention call of the T > 1 branch of

@@ -95,6 +95,31 @@ static void set_plan(DecodeParams &p, const kitty_decode_args &a, bool balanced)
     p.static_waves = plan_waves((int64_t)a.batch * a.num_kv_heads * units, p.page_waves, p.simd_waves, p.chunk_lo, p.min_chunk);
 }
 
+// The decodes the pair kernel takes: one workgroup per (sequence, KV head) pair
+// and CU, so up to resident_waves(1) pairs, of few units (pages + FP16 units)
+// each.  It saves the merge launch (and a step's append launch), and loses where
+// its 8 waves per pair leave the chip idle that the split plan fills.  Measured
+// in us, one kernel against the two, pages + 18 FP16 units:
+//   8 pairs,   20 units 12.5 / 12.9,  28 units 15.6 / 13.2
+//   64 pairs,  25 units 13.9 / 15.1,  28 units 16.5 / 15.5
+//   128 pairs, 40 units 21.1 / 21.5,  68 units 29.5 / 25.3
+//   256 pairs, 40 units 23.3 / 28.7,  68 units 34.3 / 39.9
+// and a module step (plan_pages given; host-bound up to 16 us) 16.7 / 22.6 with 8
+// pairs of 26 units, 19.2 / 22.6 of 41, 21.5 / 22.9 of 49.  A batch's units are its
+// longest sequence's, and only the split plan evens ragged ones out: at most 48.
+// A group of 16 heads (4 waves per CU: 20.8 us against 15.3) stays split.
+constexpr int kPairUnits = 21, kPairStepUnits = 44, kPairUnitsMax = 48;
+
+static bool pair_plan(const DecodeParams &p, const kitty_decode_args &a)
+{
+    const int64_t pairs = (int64_t)p.B * p.Hkv;
+    if (!p.balanced || p.GQ > 8 || a.pages_per_split != 0 || p.fp16_units <= 0 || pairs > resident_waves(1))
+        return false;
+    const int64_t pages = a.plan_pages > 0 && a.plan_pages < a.max_pages ? a.plan_pages : a.max_pages;
+    const int64_t many = std::min<int64_t>(kPairUnitsMax, 5 * pairs / 16);
+    return pages + p.fp16_units <= std::max<int64_t>(a.plan_pages > 0 ? kPairStepUnits : kPairUnits, many);
+}
+
 static void sub_group(DecodeParams &p, const kitty_decode_args &a, int s);
 
 static int build_params(const kitty_decode_args *args, DecodeParams &p)
@@ -187,6 +212,7 @@ static void sub_group(DecodeParams &p, const kitty_decode_args &a, int s)
             p.GQ = v.GQ;  // the generic kernel builds 1, 2, 4, 8 and 16 and pads the rest too
     }
     set_plan(p, a, mfma_path_supported(p));
+    p.pair = pair_plan(p, a);
 }
 
 // Partial rows of the workspace: uniform plan B * Hq * (n_splits + 1);
@@ -337,6 +363,12 @@ static int launch_decode(DecodeParams &p, const kitty_decode_args *args, kitty_s
             sub_group(p, *args, s);
             set_workspace(p, *args);
         }
+        if (p.pair) {
+            rc = launch_pair(p, StepParams{}, (hipStream_t)stream);
+            if (rc)
+                return rc;
+            continue;
+        }
         rc = launch_splits(p, (hipStream_t)stream);
         if (rc)
             return rc;
@@ -354,12 +386,27 @@ extern "C" int kitty_paged_decode(const kitty_decode_args *args, kitty_stream_t 
     return rc || p.B == 0 ? rc : launch_decode(p, args, stream);
 }
 
-extern "C" int kitty_decode_step(const kitty_append_args *append, const kitty_decode_args *decode, kitty_stream_t stream)
+// The append's buffers are the decode's, as far as the pair kernel relies on it.
+static bool step_fits(const kitty_append_args &a, const kitty_decode_args &d)
+{
+    return a.batch == d.batch && a.num_kv_heads == d.num_kv_heads && a.head_dim == d.head_dim &&
+           (a.val_len != nullptr) == (d.tail_len_v != nullptr) && a.sink_size == d.sink_capacity &&
+           a.buf_tokens == d.tail_capacity && (!a.val_len || a.val_tokens == d.tail_v_capacity);
+}
+
+extern "C" int kitty_decode_step(const kitty_append_args *append, const kitty_decode_args *decode, int32_t *tickets,
+                                 kitty_stream_t stream)
 {
     DecodeParams p;
     int rc = prepare(decode, p);
     if (rc)
         return rc;
+    if (append && tickets && p.B > 0 && p.sub_groups == 1 && p.pair && step_fits(*append, *decode)) {
+        rc = check_append(append);
+        if (rc)
+            return rc;
+        return launch_pair(p, StepParams{*append, tickets}, (hipStream_t)stream);
+    }
     rc = kitty_append_tokens(append, stream);
     return rc || p.B == 0 ? rc : launch_decode(p, decode, stream);
 }

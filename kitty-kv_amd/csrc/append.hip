@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void zero_regions_kernel(ZeroArgs a)
 
 using namespace kitty;
 
-extern "C" int kitty_append_tokens(const kitty_append_args *args, kitty_stream_t stream)
+int kitty::check_append(const kitty_append_args *args)
 {
     if (!args)
         return fail(KITTY_E_INVALID, "args is NULL");
@@ -213,7 +213,15 @@ extern "C" int kitty_append_tokens(const kitty_append_args *args, kitty_stream_t
     if (!al16(a.key) || !al16(a.value) || !al16(a.buf_k) || !al16(own_values ? a.val_buf : a.buf_v) ||
         (a.sink_size > 0 && (!al16(a.sink_k) || !al16(a.sink_v))))
         return fail(KITTY_E_INVALID, "append buffers must be 16-byte aligned");
-    hipLaunchKernelGGL(append_tokens_kernel, dim3(a.batch), dim3(64), 0, (hipStream_t)stream, a);
+    return KITTY_OK;
+}
+
+extern "C" int kitty_append_tokens(const kitty_append_args *args, kitty_stream_t stream)
+{
+    const int rc = check_append(args);
+    if (rc || args->batch == 0)
+        return rc;
+    hipLaunchKernelGGL(append_tokens_kernel, dim3(args->batch), dim3(64), 0, (hipStream_t)stream, *args);
     return check_launch("append_tokens_kernel");
 }
 

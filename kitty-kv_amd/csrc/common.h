@@ -27,6 +27,9 @@ inline int check_launch(const char *what)
     return KITTY_OK;
 }
 
+// kitty_append_tokens' checks (append.hip).
+int check_append(const kitty_append_args *args);
+
 __device__ __forceinline__ float h2f(uint16_t b)
 {
     return (float)__builtin_bit_cast(_Float16, b);

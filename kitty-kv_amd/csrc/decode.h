@@ -50,6 +50,7 @@ struct DecodeParams {
     // charged per 128 sink + tail tokens.
     int balanced, page_waves, simd_waves, chunk_lo, min_chunk, fp16_weight;
     int fp16_units;  // FP16 units per pair: seq_fp16_units(sink_cap + tail_v_cap, fp16_weight)
+    bool pair;         // few pairs of few units: one launch of decode_pair_kernel
     int static_waves;  // plan_waves of the batch with every sequence at max_pages
     float *ws_o;  // uniform: [B][Hq][num_partials][D]; balanced: [partial t][GQ][D]
     float *ws_ml; // the same rows: running max (log2 domain) and sum
@@ -74,21 +75,28 @@ struct SeqLens {
     bool bad;
 };
 
-__device__ __forceinline__ SeqLens seq_lens(const DecodeParams &p, int b)
+// Lengths as the counters give them -> checked and clamped (nk, nv: tail_len
+// and, with a value stream of its own, tail_len_v).
+__device__ __forceinline__ SeqLens check_lens(const DecodeParams &p, int ns, int npk, int npv, int nk, int nv)
 {
     SeqLens L;
-    const int npk = p.num_pages[b];
-    const int npv = p.num_pages_v ? p.num_pages_v[b] : npk;
-    const int nk = min(max(0, p.tail_len[b]), p.tail_cap);
-    const int nv = p.tail_len_v ? min(max(0, p.tail_len_v[b]), p.tail_v_cap) : nk;
+    nk = min(max(0, nk), p.tail_cap);
+    nv = p.tail_len_v ? min(max(0, nv), p.tail_v_cap) : nk;
     L.bad = npk < 0 || npk > p.max_pages || npv < 0 || npv > npk || (int64_t)(npk - npv) * p.G + nk != nv;
-    L.ns = L.bad ? 0 : min(max(0, p.sink_len[b]), p.sink_cap);
+    L.ns = L.bad ? 0 : min(max(0, ns), p.sink_cap);
     L.npk = L.bad ? 0 : npk;
     L.npv = L.bad ? 0 : npv;
     L.nk = L.bad ? 0 : nk;
     L.nv = L.bad ? 0 : nv;
     L.nmix = L.bad ? 0 : (npk - npv) * p.G;
     return L;
+}
+
+__device__ __forceinline__ SeqLens seq_lens(const DecodeParams &p, int b)
+{
+    const int npk = p.num_pages[b];
+    return check_lens(p, p.sink_len[b], npk, p.num_pages_v ? p.num_pages_v[b] : npk, p.tail_len[b],
+                      p.tail_len_v ? p.tail_len_v[b] : 0);
 }
 
 // Page count the unit plan and the page path see for sequence b: its key
@@ -180,12 +188,24 @@ __host__ __device__ inline int xcd_local_index(int i, int n)
     return n % kXcds == 0 ? (i % kXcds) * (n / kXcds) + i / kXcds : i;
 }
 
+// Waves of a pair workgroup (decode_pair_kernel): eight with 20 KB of LDS each
+// fill a CU's 160 KB.
+constexpr int kPairWaves = 8;
+
+// The append of a decode step in the pair kernel's launch; tickets NULL: no
+// append.  tickets: an int32 per slot, 0 between launches.
+struct StepParams {
+    kitty_append_args append;
+    int32_t *tickets;
+};
+
 size_t generic_lds_bytes(int GQ, int D, int G, int Dk);
 int launch_generic(const DecodeParams &p, hipStream_t stream);
 int launch_splits(const DecodeParams &p, hipStream_t stream);
 bool mfma_shape_supported(const DecodeParams &p);
 bool mfma_path_supported(const DecodeParams &p);
 int launch_mfma(const DecodeParams &p, hipStream_t stream);
+int launch_pair(const DecodeParams &p, const StepParams &step, hipStream_t stream);
 int launch_merge(const DecodeParams &p, hipStream_t stream);
 
 } // namespace kitty

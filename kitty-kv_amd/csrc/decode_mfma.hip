@@ -43,8 +43,10 @@
 // Reduction index k of every MFMA follows the natural channel / token order
 // within a 32-wide step (the tr8 row order puts even and odd bytes of a
 // word on consecutive k).
+#include <utility>
 #include "common.h"
 #include "decode.h"
+#include "merge.h"
 #include "qk_exact.h"
 
 namespace kitty {
@@ -53,7 +55,6 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef short s16x2 __attribute__((ext_vector_type(2)));
@@ -263,6 +264,24 @@ __device__ __forceinline__ unsigned pack_h2(float a, float b)
 __device__ __forceinline__ half2v as_h2(unsigned u) { return __builtin_bit_cast(half2v, u); }
 __device__ __forceinline__ unsigned as_u(half2v h) { return __builtin_bit_cast(unsigned, h); }
 
+
+// Lane of the wave (single-wave workgroups and the waves of a pair workgroup alike).
+__device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
+
+// The wave's LDS accesses so far are done before the ones that follow.  A
+// workgroup of one wave uses its barrier; the waves of a pair workgroup
+// (decode_pair_kernel) run on their own stages and wait only for themselves.
+template <bool PAIR>
+__device__ __forceinline__ void wave_sync()
+{
+    if constexpr (PAIR) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
 
 struct PageSrc {
     const unsigned char *klo, *val, *khi, *kmeta, *vmeta;
@@ -888,7 +907,7 @@ template <int GQ>
 __device__ __forceinline__ SegSetup load_setup(const DecodeParams &p, int b, int kh, int p0, int p1)
 {
     constexpr int ROWS_PER_HEAD = 16 / GQ;
-    const int lane = threadIdx.x, q = lane >> 4, r = lane & 15;
+    const int lane = lane_id(), q = lane >> 4, r = lane & 15;
     SegSetup s;
     s.bi0 = p.boost_idx[kh * 128 + lane];
     s.bi1 = p.boost_idx[kh * 128 + 64 + lane];
@@ -909,7 +928,7 @@ __device__ __forceinline__ SegSetup load_setup(const DecodeParams &p, int b, int
 // above its largest |q| (exact for every channel within 2^-23 of that), and
 // the scores take 2^(E - 9) back: with page scales below 16 the operands stay
 // below 2^13, 2^15 on the high-bit rows.
-template <int GQ, bool BF>
+template <int GQ, bool BF, bool PAIR = false>
 __device__ __forceinline__ void qk_setup(WaveState<GQ, BF> &W, const DecodeParams &p, int b, int kh, const SegSetup &su,
                                          unsigned char *scratch, int lane, int Dk)
 {
@@ -926,7 +945,7 @@ __device__ __forceinline__ void qk_setup(WaveState<GQ, BF> &W, const DecodeParam
     _Float16 *q_lds = (_Float16 *)(scratch + 256);  // [GQ][128]
     if (lane < 32)
         rank_chan[lane] = 0;
-    __syncthreads();
+    wave_sync<PAIR>();
     if (su.bi0 < Dk)
         rank_chan[su.bi0] = lane;
     if (su.bi1 < Dk)
@@ -937,7 +956,7 @@ __device__ __forceinline__ void qk_setup(WaveState<GQ, BF> &W, const DecodeParam
             *(u32x4 *)(q_lds + hr * 128 + 32 * s + 8 * q) = su.qraw[s];
     }
 
-    __syncthreads();
+    wave_sync<PAIR>();
 
     // Static half of the QK A operand: 2^-3 q (fp16) of the lane's 8 channels
     // of every K-step on the two rows of each head (the product with the key
@@ -1022,7 +1041,8 @@ __device__ __forceinline__ void qk_setup(WaveState<GQ, BF> &W, const DecodeParam
 // holds query head kh * GQ + h.  A page count outside [0, max_pages] or a
 // page id outside the pool makes the partial NaN; no pages leave an empty
 // partial (m = -inf, l = 0, O = 0).
-template <int GQ, bool BF>
+// PAIR: su.ids holds the block table's first 64 entries instead of those from p0.
+template <int GQ, bool BF, bool PAIR = false>
 __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned char *stage0, unsigned char *stage1,
                                              int b, int kh, int np_raw, int p0, int p1, int64_t t, const SegSetup &su)
 {
@@ -1030,7 +1050,7 @@ __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned cha
     constexpr int RSTEP = 4 / HPL;
     // lane-derived offsets are rebuilt per segment (the asm hides the lane
     // id): kept across the caller's segment loop they would be spilled
-    int lane = threadIdx.x;
+    int lane = lane_id();
     asm volatile("" : "+v"(lane));
     const int q = lane >> 4, r = lane & 15;
     const int Dk = p.Dk;
@@ -1047,7 +1067,7 @@ __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned cha
         p1 = np_raw;
 
     WaveState<GQ, BF> W;
-    qk_setup<GQ, BF>(W, p, b, kh, su, stage1, lane, Dk);
+    qk_setup<GQ, BF, PAIR>(W, p, b, kh, su, stage1, lane, Dk);
     // tr4 offsets of value rows R = 32q + 16k + r (GQA 4): 16-byte chunk c of
     // row R sits at 32 R + 16 (c ^ ((R >> 3) & 1)) in the stage.
 #pragma unroll
@@ -1079,7 +1099,7 @@ __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned cha
 #pragma unroll
     for (int ch = 0; ch < 4; ++ch)
         W.o4[ch][0] = W.o4[ch][1] = 0.0f;
-    __syncthreads();  // stage1 reads done before the next page lands there
+    wave_sync<PAIR>();  // stage1 reads done before the next page lands there
 
     // Page ids, 64 at a time (one per lane), read back with v_readlane so no
     // page waits on a dependent global load; pages are asked for in order,
@@ -1088,10 +1108,12 @@ __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned cha
     // pages): left pending, it would make the compiler wait for every
     // outstanding load before each page's v_readlane.
     const int32_t *bt = p.block_table + b * p.bt_stride;
-    int chunk0 = p0;
+    int chunk0 = PAIR ? 0 : p0;
     int ids = su.ids;
     auto page_ok = [&](int32_t page) { return page >= 0 && page < p.num_pool_pages; };
     auto page_at = [&](int pi) -> int32_t {
+        while (PAIR && pi - chunk0 >= 128)
+            chunk0 += 64;
         if (pi - chunk0 >= 64) {
             chunk0 += 64;
             ids = chunk0 + lane < p1 ? bt[chunk0 + lane] : 0;
@@ -1192,7 +1214,7 @@ __device__ __forceinline__ void page_segment(const DecodeParams &p, unsigned cha
 template <int GQ>
 __device__ __forceinline__ void empty_partial(const DecodeParams &p, int64_t t)
 {
-    const int lane = threadIdx.x;
+    const int lane = lane_id();
 #pragma unroll
     for (int g = 0; g < GQ; ++g) {
         const int64_t row = t * GQ + g;
@@ -1268,59 +1290,93 @@ __device__ __forceinline__ DecodeParams kernel_params(KernargParams pp)
     return r;
 }
 
-// FP16-region tokens [lo, hi) of pair (b, kh), 32 per step.  The region is
-// the sinks, then the tokens of the key-only pages P_v .. P_k - 1 (an
+// FP16-region tokens [lo, hi) of pair (b, kh), 32 per step, as partial t.  The
+// region is the sinks, then the tokens of the key-only pages P_v .. P_k - 1 (an
 // independent value stream: their keys are quantised, their values are the
 // first (P_k - P_v) G rows of the value tail), then the key tail, whose
 // values follow in the value tail; with one stream the middle part is empty.
 // A step's rows stream into the two LDS stages with global_load_lds (no
 // registers hold data in flight): K chunk c of token row n is stored at
 // chunk c ^ (n & 15), so the 16 rows one MFMA B read touches hit 16
-// different bank groups.  QK: f16 MFMAs with the heads on rows (A = q,
-// B = K rows, exact products; scores times sm_scale log2(e) in fp32); for a
-// key-only page the page path's exact QK (page_qk) writes the page's scores
-// to kst once and its steps read them back.  Base-2 online softmax per head
-// row with DPP row reductions, P through LDS.  PV: VALU, lane = channel
-// pair.  Steps do not cross from sinks into key-only pages, nor out of one.
-// Returns each head's (m, l) and O (channels 2 lane, 2 lane + 1); m is NaN
-// if a key-only page id lies outside the pool.
-template <int GQ, bool BF>
-__device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int hi, unsigned char *kst,
-                              unsigned char *vst, float *m_out, float *l_out, float (*O)[2])
+// different bank groups; V rows lie as they are.  QK: f16 or bf16 MFMAs
+// with head h on rows 16 / GQ h .. (A = q, B = K rows, exact products; scores
+// times sm_scale log2(e) in fp32), so a lane holds the scores of its group's
+// GQ / 4 heads; for a key-only page the page path's exact QK (page_qk) writes
+// the page's scores to kst once and its steps read them back.  Base-2 online
+// softmax per head with DPP row reductions.  PV: fp32 MFMAs of 4 heads x 1 token
+// x 4 channels in 16 blocks, whose columns are the lanes in order: a lane holds a
+// channel pair, one MFMA does a token, 4 heads and one channel of every pair.
+// One register holds P of 16 tokens x 4 heads, a token's block broadcast to all.
+// (16-bit terms of P in 16 x 16 x 32 MFMAs were as fast, but their products are
+// aligned to the largest and truncated: rms error of the output against 64 bits
+// 8e-8 where fp32 has 2.4e-8.)
+// Steps do not cross from sinks into key-only pages, nor out of one.  The
+// partial's m is NaN if a key-only page id lies outside the pool.
+// Bound by its chain of loads, MFMAs and softmax per step, not by the units:
+// PV on the VALU (lane = channel pair, fp32 P) and four scores per lane for
+// every group took 15.8 us where this takes 13.5 (1 x 1,024 tokens, pair
+// kernel) and 22.3 against 21.6 (8 x 3-9K tokens, bf16, split).  q is loaded
+// again by every step: kept, with 16-bit terms, the split kernel spilled 25-43
+// registers (16 x 32K tokens: 80 us instead of 66), and even 8 spilled ones cost
+// 4 x 128K tokens, groups of 8, 2 us of 76.
+//
+// L: the sequence's lengths.  Token nt.last (PAIR only) is the one this step
+// appends: its rows are read from the step's inputs.
+struct NewToken {
+    const uint16_t *k, *v;
+    int last;  // its index in the region, -1: none
+};
+
+// O += P V of 16 tokens: the lane's channel pair of each in x, P of head group
+// g at pb + 128 g.
+template <int GQ, bool BF, int... T>
+__device__ __forceinline__ void pv16(f32x4 (&O)[GQ / 4][2], const float *pb, const uint32_t *x, int lane,
+                                     std::integer_sequence<int, T...>)
+{
+    float pr[GQ / 4];
+#pragma unroll
+    for (int g = 0; g < GQ / 4; ++g)
+        pr[g] = pb[128 * g + lane];
+    auto token = [&](auto tc) {
+        constexpr int tok = decltype(tc)::value;
+        const float v0 = BF ? bf2f((uint16_t)x[tok]) : h2f((uint16_t)x[tok]);
+        const float v1 = BF ? bf2f((uint16_t)(x[tok] >> 16)) : h2f((uint16_t)(x[tok] >> 16));
+#pragma unroll
+        for (int g = 0; g < GQ / 4; ++g) {
+            O[g][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(pr[g], v0, O[g][0], 4, tok, 0);
+            O[g][1] = __builtin_amdgcn_mfma_f32_4x4x1f32(pr[g], v1, O[g][1], 4, tok, 0);
+        }
+    };
+    (token(std::integral_constant<int, T>{}), ...);
+}
+
+template <int GQ, bool BF, bool PAIR>
+__device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int hi, int64_t t, const SeqLens &L,
+                              const NewToken &nt, unsigned char *kst, unsigned char *vst)
 {
     constexpr int kTok = 32;
-    constexpr int HPL = GQ / 4;
-    constexpr int RSTEP = 4 / HPL;
-    const int lane = threadIdx.x, r = lane & 15, kq = lane >> 4;
-    float *pbuf = (float *)(vst + kTok * 256);  // [head][token] fp32, GQ * 32 floats
-    // A operand: row r = head r (rows past GQ are zero), k = 8 kq + i of each
-    // 32-channel step
-    // (fp16 q as is: q k is exact in the fp32 accumulator, and the scores
+    constexpr int HPL = GQ / 4;              // heads per lane group
+    constexpr int RSTEP = 4 / HPL;           // accumulator register of head slot j = j * RSTEP
+    constexpr int RPH = 16 / GQ;             // MFMA rows per head
+    constexpr int NG = GQ / 4;               // groups of 4 heads
+    const int lane = lane_id(), r = lane & 15, kq = lane >> 4;
+    static_assert(kTok * 256 + GQ * kTok * 4 <= kStage, "P does not fit behind the value rows");
+    float *pbuf = (float *)(vst + kTok * 256);  // P[head / 4][token][head % 4]
+    // A operand: row r = head r / RPH, k = 8 kq + i of each 32-channel step
+    // (q as is: q k is exact in the fp32 accumulator, and the scores
     // are scaled by sm_scale log2(e) afterwards)
-    half8 qa[4];
+    const uint16_t *qrow = p.q + b * p.q_s_seq + q_head(p, kh, r / RPH) * p.q_s_head + 8 * kq;
     const float qk_c = p.sm_scale * kLog2e;
-    {
-        const uint16_t *qrow = p.q + b * p.q_s_seq + q_head(p, kh, r < GQ ? r : 0) * p.q_s_head;
+    float m[HPL], l[HPL];  // head kq HPL + j; l: this lane's tokens
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const u32x4 raw = *(const u32x4 *)(qrow + 32 * s + 8 * kq);
-            u32x4 v;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                v[j] = r < GQ ? raw[j] : 0u;
-            qa[s] = __builtin_bit_cast(half8, v);
-        }
+    for (int j = 0; j < HPL; ++j) {
+        m[j] = -__builtin_inff();
+        l[j] = 0.0f;
     }
-    float m[4], l[4];  // head rows 4 kq + i
+    f32x4 O[NG][2];        // heads 4 g + i, channels 2 lane + c
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        m[i] = -__builtin_inff();
-        l[i] = 0.0f;
-    }
-#pragma unroll
-    for (int g = 0; g < GQ; ++g)
-        O[g][0] = O[g][1] = 0.0f;
-    const SeqLens L = seq_lens(p, b);
+    for (int g = 0; g < NG; ++g)
+        O[g][0] = O[g][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const int ns = L.ns, kbeg = L.ns, kend = L.ns + L.nmix;  // key-only tokens [kbeg, kend)
     const uint16_t *sk = p.sink_k.ptr + b * p.sink_k.s_seq + kh * p.sink_k.s_head;
     const uint16_t *sv = p.sink_v.ptr + b * p.sink_v.s_seq + kh * p.sink_v.s_head;
@@ -1338,7 +1394,7 @@ __device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int 
         else if (c0 < kbeg && kend > kbeg)
             end = min(end, kbeg);
         const int cnt = end - c0;
-        f32x4 S[2];
+        float S[2][HPL];
         if (konly) {
             if (pg != page_in_kst) {
                 // scores of key page P_v + pg: the page path's QK into kst
@@ -1350,13 +1406,12 @@ __device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int 
                 }
                 WaveState<GQ, BF> W;
                 const SegSetup su = load_setup<GQ>(p, b, kh, L.npv + pg, L.npv + pg + 1);
-                qk_setup<GQ, BF>(W, p, b, kh, su, vst, lane, p.Dk);
+                qk_setup<GQ, BF, PAIR>(W, p, b, kh, su, vst, lane, p.Dk);
                 issue_page(kst, page_src(p, (int64_t)page * p.Hkv + kh), lane, p.Dk);
                 wait_vmcnt<0>();
                 f32x4 Sp[2][4], Yt;
                 float kmul;
                 page_qk<GQ, BF>(W, kst, lane, p.Dk, Sp, Yt, kmul);
-                const int q = kq;
                 float *scw = (float *)kst;
 #pragma unroll
                 for (int j = 0; j < HPL; ++j) {
@@ -1368,11 +1423,11 @@ __device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int 
                     for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
                         for (int a = 0; a < 4; ++a)
-                            scw[(q * HPL + j) * 128 + 64 * cb + 4 * r + a] =
+                            scw[(kq * HPL + j) * 128 + 64 * cb + 4 * r + a] =
                                 (GQ == 16 ? Sp[cb][a][ri] : Sp[cb][a][ri] + Sp[cb][a][ri + 1]) *
                                     (page_c * (kSub / slot_weight<BF>(a))) - yk;
                 }
-                __syncthreads();  // scores in kst before they are read back
+                wave_sync<PAIR>();  // scores in kst before they are read back
                 page_in_kst = pg;
             }
             // ---- value rows of the step: value-tail rows c0 - ns ..
@@ -1387,11 +1442,15 @@ __device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int 
 #pragma unroll
             for (int tg = 0; tg < 2; ++tg)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int h = 4 * kq + i, t = 16 * tg + r;
-                    S[tg][i] = h < GQ && t < cnt ? sc[h * 128 + t0 + t] : 0.0f;
+                for (int j = 0; j < HPL; ++j) {
+                    const int tok = 16 * tg + r;
+                    S[tg][j] = tok < cnt ? sc[(kq * HPL + j) * 128 + t0 + tok] : -__builtin_inff();
                 }
         } else {
+            u32x4 qa[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                qa[s] = *(const u32x4 *)(qrow + 32 * s);
             // ---- 16 direct-to-LDS loads: instruction i covers rows 4i .. 4i+3
 #pragma unroll
             for (int i = 0; i < kTok / 4; ++i) {
@@ -1402,88 +1461,84 @@ __device__ void fp16_segments(const DecodeParams &p, int b, int kh, int lo, int 
                                             : tk + (int64_t)(tt - kend) * p.tail_k.s_tok;
                 const uint16_t *vrow = sink ? sv + (int64_t)tt * p.sink_v.s_tok
                                             : tv + (int64_t)(tt - ns) * p.tail_v.s_tok;
+                if (PAIR && tt == nt.last) {
+                    krow = nt.k;
+                    vrow = nt.v;
+                }
                 gll16((const unsigned char *)(krow + 8 * (r ^ (n & 15))), kst + 1024 * i);
                 gll16((const unsigned char *)(vrow + 8 * r), vst + 1024 * i);
             }
             wait_vmcnt<0>();
-            // ---- QK: tile tg covers tokens 16 tg + r; S[tg][i] = head 4 kq + i
+            // ---- QK: tile tg covers tokens 16 tg + r
 #pragma unroll
             for (int tg = 0; tg < 2; ++tg) {
-                S[tg] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 const int n = 16 * tg + r;
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    const half8 kb = *(const half8 *)(kst + 256 * n + 16 * ((4 * s + kq) ^ r));
+                    const u32x4 kb = *(const u32x4 *)(kst + 256 * n + 16 * ((4 * s + kq) ^ r));
                     if constexpr (BF)
-                        S[tg] = mfma_bf(__builtin_bit_cast(bf16x8, qa[s]), __builtin_bit_cast(bf16x8, kb), S[tg]);
+                        acc = mfma_bf(__builtin_bit_cast(bf16x8, qa[s]), __builtin_bit_cast(bf16x8, kb), acc);
                     else
-                        S[tg] = mfma(qa[s], kb, S[tg]);
+                        acc = mfma(__builtin_bit_cast(half8, qa[s]), __builtin_bit_cast(half8, kb), acc);
                 }
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    S[tg][i] *= qk_c;
+                for (int j = 0; j < HPL; ++j)
+                    S[tg][j] = n < cnt ? acc[j * RSTEP] * qk_c : -__builtin_inff();
             }
             page_in_kst = -1;  // K rows went over any page scores
         }
-        // ---- online softmax per head row (tokens past cnt masked)
-        float alpha[4];
+        // the step's values, ahead of the softmax: read two at a time between the
+        // MFMAs they cost an LDS round trip each
+        uint32_t x[kTok];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float s0 = r < cnt ? S[0][i] : -__builtin_inff();
-            const float s1 = 16 + r < cnt ? S[1][i] : -__builtin_inff();
-            const float mx = row_max16(fmaxf(s0, s1));
-            const float mn = fmaxf(m[i], mx);
-            alpha[i] = __builtin_amdgcn_exp2f(m[i] - mn);
-            const float p0 = __builtin_amdgcn_exp2f(s0 - mn), p1 = __builtin_amdgcn_exp2f(s1 - mn);
-            l[i] = l[i] * alpha[i] + row_sum16(p0 + p1);
-            m[i] = mn;
-            const int h = 4 * kq + i;
-            if (h < GQ) {
-                pbuf[h * kTok + r] = p0;
-                pbuf[h * kTok + 16 + r] = p1;
-            }
-        }
-        __syncthreads();
-        // ---- PV: lane = channels 2 lane, 2 lane + 1
+        for (int n = 0; n < kTok; ++n)
+            x[n] = *(const uint32_t *)(vst + 256 * n + 4 * lane);
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- online softmax per head (tokens past cnt masked), P to LDS
+        float alpha[HPL];
 #pragma unroll
-        for (int g = 0; g < GQ; ++g) {
-            const float al = __builtin_bit_cast(
-                float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, alpha[g & 3]), 16 * (g >> 2)));
-            O[g][0] *= al;
-            O[g][1] *= al;
+        for (int j = 0; j < HPL; ++j) {
+            const float mn = fmaxf(m[j], row_max16(fmaxf(S[0][j], S[1][j])));
+            alpha[j] = __builtin_amdgcn_exp2f(m[j] - mn);
+            m[j] = mn;
+            const float p0 = __builtin_amdgcn_exp2f(S[0][j] - mn), p1 = __builtin_amdgcn_exp2f(S[1][j] - mn);
+            l[j] = l[j] * alpha[j] + (p0 + p1);
+            const int h = kq * HPL + j;
+            float *ph = pbuf + (h >> 2) * (4 * kTok) + (h & 3);
+            ph[4 * r] = p0;
+            ph[4 * (16 + r)] = p1;
         }
 #pragma unroll
-        for (int t4 = 0; t4 < kTok / 4; ++t4) {
-            unsigned vv[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                vv[e] = *(const unsigned *)(vst + 256 * (4 * t4 + e) + 4 * lane);
-#pragma unroll
-            for (int g = 0; g < GQ; ++g) {
-                const float4 w = *(const float4 *)(pbuf + g * kTok + 4 * t4);
-                const float wt[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const half2v h = as_h2(vv[e]);
-                    O[g][0] += wt[e] * (BF ? bf_lo(vv[e]) : (float)h[0]);
-                    O[g][1] += wt[e] * (BF ? bf_hi(vv[e]) : (float)h[1]);
-                }
-            }
+        for (int h = 0; h < GQ; ++h) {  // the head's alpha from its lane group
+            const float x = __builtin_bit_cast(
+                float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, alpha[h % HPL]), 16 * (h / HPL)));
+            O[h / 4][0][h % 4] *= x;
+            O[h / 4][1][h % 4] *= x;
         }
-        __syncthreads();  // LDS reads done before the next step's loads land
+        wave_sync<PAIR>();
+        // ---- PV, 16 tokens per P register
+        pv16<GQ, BF>(O, pbuf, x, lane, std::make_integer_sequence<int, 16>{});
+        if (cnt > 16)
+            pv16<GQ, BF>(O, pbuf + 64, x + 16, lane, std::make_integer_sequence<int, 16>{});
+        wave_sync<PAIR>();  // LDS reads done before the next step's loads land
         c0 = end;
     }
 #pragma unroll
-    for (int g = 0; g < GQ; ++g) {
-        m_out[g] = poison ? __builtin_nanf("")
-                          : __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m[g & 3]), 16 * (g >> 2)));
-        l_out[g] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, l[g & 3]), 16 * (g >> 2)));
+    for (int j = 0; j < HPL; ++j) {
+        const float lsum = row_sum16(l[j]);
+        if (r == 0) {
+            const int64_t row = t * GQ + kq * HPL + j;
+            p.ws_ml[2 * row] = poison ? __builtin_nanf("") : m[j];
+            p.ws_ml[2 * row + 1] = lsum;
+        }
     }
+#pragma unroll
+    for (int h = 0; h < GQ; ++h)
+        *(float2 *)(p.ws_o + (t * GQ + h) * 128 + 2 * lane) = make_float2(O[h / 4][0][h % 4], O[h / 4][1][h % 4]);
 }
 
-
-// FP16 tokens [lo, hi) of pair (b, kh) as partial t.  Out of line: the page
-// loop's registers need not be kept around it.
+// FP16 tokens [lo, hi) of pair (b, kh) as partial t.
 template <int GQ, bool BF>
 __device__ __forceinline__ void fp16_partial(KernargParams kp, int b, int kh, int lo, int hi, int64_t t,
                                           unsigned char *stage0, unsigned char *stage1)
@@ -1496,17 +1551,7 @@ __device__ __forceinline__ void fp16_partial(KernargParams kp, int b, int kh, in
     kh = __builtin_amdgcn_readfirstlane(kh);
     lo = __builtin_amdgcn_readfirstlane(lo);
     hi = __builtin_amdgcn_readfirstlane(hi);
-    const int lane = threadIdx.x;
-    float m[GQ], l[GQ], O[GQ][2];
-    fp16_segments<GQ, BF>(P, b, kh, lo, hi, stage0, stage1, m, l, O);
-    for (int g = 0; g < GQ; ++g) {
-        const int64_t row = t * GQ + g;
-        *(float2 *)(P.ws_o + row * 128 + 2 * lane) = make_float2(O[g][0], O[g][1]);
-        if (lane == 0) {
-            P.ws_ml[2 * row] = m[g];
-            P.ws_ml[2 * row + 1] = l[g];
-        }
-    }
+    fp16_segments<GQ, BF, false>(P, b, kh, lo, hi, t, seq_lens(P, b), NewToken{nullptr, nullptr, -1}, stage0, stage1);
     __syncthreads();  // stage reads done before the next segment reuses them
 }
 
@@ -1655,6 +1700,7 @@ void decode_mfma_kernel(DecodeParams p)
             fp16_partial<GQ, BF>(kp, sq.b, kh, fa * ntok / F, fc * ntok / F, (int64_t)w + 2 * j + 1, stage0, stage1);
             u = e;
         }
+        spec = SegSetup{};  // dead from here: its registers are the walk's
         if (u == s_j + per_pair && lane == 0)  // this wave ends the pair: its last partial
             kernel_params(kp).ws_pair[2 * j + 1] = w + 2 * j + (F > 0 ? 1 : 0);
         if (u >= u_end)
@@ -1666,6 +1712,115 @@ void decode_mfma_kernel(DecodeParams p)
             sq.base += Hkv * per_pair;
             sq.np_raw = seq_np_raw(P, sq.b);
             sq.npu = seq_page_units(sq.np_raw, P.max_pages, F);
+        }
+    }
+}
+
+// Decode of batches with few pairs of few units in one launch: one workgroup
+// per (sequence, KV head) pair, whose waves each take an equal run of the
+// pair's units (pages, then FP16 units) on stages of their own, write their
+// partials, and after one barrier merge them, a head per wave.  With `step`
+// the launch also appends the step's token: its rows are stored to the buffers
+// and attended from the inputs, and the last workgroup of a sequence to finish
+// (step.tickets) advances its counters, which every workgroup has read by then.
+//
+// Such a decode is bound by its chain of launches and dependent loads, not by
+// the chip: a split launch (plan over all sequences, then the first segment),
+// a merge launch, and the append launch before them.  The lengths, q, ranks and
+// page ids are one round trip here.  1 x 512 tokens, 8 KV heads: 11.2 us against
+// 12.0 of the split and merge launches (16.9 with an FP16 walk on the VALU); a
+// module step of 1 x 1,000 tokens 16.0 us against 20.4, of 16 x 1,000 tokens and
+// 8 KV heads 21.3 against 26.0.
+template <int GQ, bool BF>
+__global__ __launch_bounds__(64 * kPairWaves) __attribute__((amdgpu_waves_per_eu(2)))
+void decode_pair_kernel(DecodeParams p, StepParams step)
+{
+    constexpr int NW = kPairWaves;
+    __shared__ __attribute__((aligned(16))) unsigned char stage0[NW][kStage];
+    __shared__ __attribute__((aligned(16))) unsigned char stage1[NW][kStage];
+    const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int pair = blockIdx.x, b = pair / p.Hkv, kh = pair - b * p.Hkv;
+
+    // ---- lengths as they stand, then (with a step) as this token leaves them
+    int ns = p.sink_len[b], nk = p.tail_len[b], npk = p.num_pages[b];
+    int npv = p.num_pages_v ? p.num_pages_v[b] : npk, nv = p.tail_len_v ? p.tail_len_v[b] : nk;
+    const SegSetup su = load_setup<GQ>(p, b, kh, 0, p.max_pages);
+    bool fresh = false, to_sink = false;
+    int slot = 0;
+    if (step.tickets) {
+        const kitty_append_args &a = step.append;
+        slot = a.slots[b];
+        to_sink = ns < a.sink_size;
+        fresh = slot >= 0 && slot < a.num_slots &&
+                (to_sink || !(nk >= a.buf_tokens || (a.val_len && nv >= a.val_tokens)));
+    }
+    const int ns0 = ns, nk0 = nk, nv0 = nv;
+    if (fresh) {
+        ns += to_sink ? 1 : 0;
+        nk += to_sink ? 0 : 1;
+        nv += to_sink ? 0 : 1;
+    }
+    const SeqLens L = check_lens(p, ns, npk, npv, nk, nv);
+    NewToken nt{nullptr, nullptr, -1};
+    if (fresh) {
+        const kitty_append_args &a = step.append;
+        nt.k = a.key + b * a.key_s_seq + kh * a.key_s_head;
+        nt.v = a.value + b * a.value_s_seq + kh * a.value_s_head;
+        nt.last = to_sink ? L.ns - 1 : L.ns + L.nv - 1;
+        if (wave == 0 && lane < 32) {   // its rows into the buffers: lanes 0-15 the key, 16-31 the value
+            const bool v = lane >= 16;
+            const kitty_slot_layout KL = to_sink ? a.sink_layout : (v && a.val_len ? a.val_layout : a.buf_layout);
+            uint16_t *dst = to_sink ? (v ? a.sink_v : a.sink_k) : (v ? (a.val_len ? a.val_buf : a.buf_v) : a.buf_k);
+            const int row = to_sink ? ns0 : (v && a.val_len ? nv0 : nk0);
+            *(u32x4 *)(dst + slot * KL.s_slot + kh * KL.s_head + row * KL.s_tok + 8 * (lane & 15)) =
+                *(const u32x4 *)((v ? nt.v : nt.k) + 8 * (lane & 15));
+        }
+    }
+    // ---- wave w takes units [w U / NW, (w + 1) U / NW) of the pair (none where
+    // the two meet); waves [0, wp) start in the pages, waves [wf, NW) end past them
+    const int F = p.fp16_units;
+    const int npu = __builtin_amdgcn_readfirstlane(L.npv);
+    const unsigned U = npu + F;
+    const int ua = wave * U / NW, ue = (wave + 1) * U / NW;
+    int wp = 0, wf = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        wp += (int)(w * U / NW) < npu ? 1 : 0;
+        wf += (int)((w + 1) * U / NW) <= npu ? 1 : 0;
+    }
+    const int64_t t0 = (int64_t)pair * (2 * NW);
+    if (ua < npu && !L.bad)
+        page_segment<GQ, BF, true>(p, stage0[wave], stage1[wave], b, kh, npu, ua, ue < npu ? ue : npu, t0 + wave, su);
+    if (wave >= wf) {
+        const int fa = (ua > npu ? ua : npu) - npu, fc = ue - npu;
+        const unsigned ntok = __builtin_amdgcn_readfirstlane(L.ns + L.nv);  // F is a few dozen here
+        wave_sync<true>();
+        fp16_segments<GQ, BF, true>(p, b, kh, (int)(fa * ntok / (unsigned)F), (int)(fc * ntok / (unsigned)F),
+                                    t0 + wp + (wave - wf), L, nt, stage0[wave], stage1[wave]);
+    }
+    __syncthreads();
+    for (int g = wave; g < p.gq; g += NW) {
+        uint16_t *o = p.out + b * p.out_s_seq + ((int64_t)kh * p.gq_stride + g) * p.out_s_head;
+        if (L.bad) {
+            o[2 * lane] = o[2 * lane + 1] = out_bits(p, __builtin_nanf(""));
+            continue;
+        }
+        merge_quads<3>(p, t0 * GQ + g, GQ, wp + NW - wf, o);
+    }
+    if (step.tickets && threadIdx.x == 0) {
+        const kitty_append_args &a = step.append;
+        // the last of the sequence's Hkv workgroups; the ticket wraps to 0 with it
+        if (slot >= 0 && slot < a.num_slots &&
+            atomicInc((unsigned *)step.tickets + slot, (unsigned)p.Hkv - 1) == (unsigned)p.Hkv - 1) {
+            if (!fresh) {
+                a.overflow[b] = 1;
+            } else if (to_sink) {
+                a.sink_fill[slot] = ns0 + 1;
+            } else {
+                a.buf_len[slot] = nk0 + 1;
+                if (a.val_len)
+                    a.val_len[slot] = nv0 + 1;
+            }
         }
     }
 }
@@ -1698,6 +1853,26 @@ static void launch_group(const DecodeParams &p, hipStream_t stream)
         hipLaunchKernelGGL((decode_mfma_kernel<GQ, true>), grid, dim3(64), 0, stream, p);
     else
         hipLaunchKernelGGL((decode_mfma_kernel<GQ, false>), grid, dim3(64), 0, stream, p);
+}
+
+template <int GQ>
+static void launch_pair_group(const DecodeParams &p, const StepParams &step, hipStream_t stream)
+{
+    const dim3 grid((unsigned)(p.B * p.Hkv)), block(64 * kPairWaves);
+    if (p.act_bf16)
+        hipLaunchKernelGGL((decode_pair_kernel<GQ, true>), grid, block, 0, stream, p, step);
+    else
+        hipLaunchKernelGGL((decode_pair_kernel<GQ, false>), grid, block, 0, stream, p, step);
+}
+
+int launch_pair(const DecodeParams &p, const StepParams &step, hipStream_t stream)
+{
+    switch (p.GQ) {
+    case 4: launch_pair_group<4>(p, step, stream); break;
+    case 8: launch_pair_group<8>(p, step, stream); break;
+    default: return fail(KITTY_E_UNSUPPORTED, "the pair kernel needs a GQA group of 4 or 8");
+    }
+    return check_launch("decode_pair_kernel");
 }
 
 int launch_mfma(const DecodeParams &p, hipStream_t stream)

@@ -96,6 +96,7 @@ class DecodeArgs(ctypes.Structure):
         ("workspace", _vp), ("workspace_bytes", ctypes.c_size_t),
         ("num_pages_v", _vp), ("tail_len_v", _vp), ("tail_v_capacity", _i32),
         ("meta_dtype", _i32), ("act_dtype", _i32), ("out_dtype", _i32),
+        ("plan_pages", _i32),
     ]
 
 
@@ -203,7 +204,7 @@ def load() -> ctypes.CDLL:
     L.kitty_channel_abs_sum_first.argtypes = [_vp, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t,
                                               _vp]
     L.kitty_channel_scores.argtypes = [ctypes.POINTER(ScoreLayer), _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp]
-    L.kitty_decode_step.argtypes = [ctypes.POINTER(AppendArgs), ctypes.POINTER(DecodeArgs), _vp]
+    L.kitty_decode_step.argtypes = [ctypes.POINTER(AppendArgs), ctypes.POINTER(DecodeArgs), _vp, _vp]
     L.kitty_store_prompt.argtypes = [ctypes.POINTER(PromptArgs), _vp]
     L.kitty_zero_regions.argtypes = [ctypes.POINTER(ZeroRegion), _i32, _vp]
     L.kitty_prefill_attention.argtypes = [ctypes.POINTER(PrefillArgs), _vp]

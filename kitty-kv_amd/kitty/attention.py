@@ -107,11 +107,14 @@ class KittyPagedAttention(nn.Module):
             out = torch.empty_like(q)
             args = hit[1].step_args(q, out)
             if not pipe._push(self.layer_id, k[:, :, 0], v[:, :, 0], ids, args):
+                args.plan_pages = pipe._longest(self.layer_id, pipe._slots(ids))
                 hit[1].run_args(args)
             return out
         pipe.push_tokens(self.layer_id, k[:, :, 0], v[:, :, 0], seq_ids)
         qd = q[:, :, 0].to(pipe.buffer_dtype).contiguous()
         plan = self._plan(qd, seq_ids)
+        if isinstance(plan, DecodePlan):
+            plan.args.plan_pages = pipe._longest(self.layer_id, pipe._slots(ids))   # as the steps in one call
         if isinstance(plan, DecodePlan) and tuple(pipe.slot(s) for s in seq_ids) in self._plans:
             if len(self._steps) >= 64:
                 self._steps.clear()

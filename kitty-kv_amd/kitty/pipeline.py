@@ -104,6 +104,7 @@ class KittyInferencePipeline:
         # device counters (kind, layer, slot): a (layer, slot range) is a contiguous (B,) int32 view
         self.lens = torch.zeros(5, L, n, dtype=torch.int32, device=dev)
         self._overflow = torch.zeros(n, dtype=torch.int32, device=dev)
+        self._tickets = torch.zeros(L, n, dtype=torch.int32, device=dev)   # kitty_decode_step's, 0 between calls
         self.max_pages_per_seq = (config.max_seq_len - S) // G + 2
         self._block_table = torch.zeros(L, n, self.max_pages_per_seq, dtype=torch.int32, device=dev)
         self._pages = np.zeros((n, L, self.max_pages_per_seq), np.int64)   # host mirror of the block table
@@ -229,14 +230,7 @@ class KittyInferencePipeline:
         """One token for each of B sequences: keys / values (B, num_kv_heads, head_dim)."""
         self._push(layer_id, keys, values, seq_ids, None)
 
-    def _push(self, layer_id: int, keys: torch.Tensor, values: torch.Tensor, seq_ids: Sequence[int],
-              decode: Optional[_hip.DecodeArgs]) -> bool:
-        """push_tokens; with the arguments of the decode that follows, a token
-        that fills no buffer is appended and decoded by one kitty_decode_step
-        call.  True when it was (a spill comes between the two otherwise)."""
-        cfg = self.config
-        S, G = cfg.sink_size, cfg.q_buffer_size
-        ids = tuple(seq_ids)
+    def _slots(self, ids: Tuple[int, ...]) -> np.ndarray:
         slots = self._slots_of_ids.get(ids)
         if slots is None:
             slots = np.array([self.slot(s) for s in ids], np.int64)
@@ -245,6 +239,23 @@ class KittyInferencePipeline:
             if len(self._slots_of_ids) >= 256:
                 self._slots_of_ids.clear()
             self._slots_of_ids[ids] = slots
+        return slots
+
+    def _longest(self, layer_id: int, slots: np.ndarray) -> int:
+        """kitty_decode_args.plan_pages of these slots' next decode."""
+        return max(1, int(self._npages[slots, layer_id].max()) if len(slots) != 1 else int(self._npages[slots[0], layer_id]))
+
+    def _push(self, layer_id: int, keys: torch.Tensor, values: torch.Tensor, seq_ids: Sequence[int],
+              decode: Optional[_hip.DecodeArgs]) -> bool:
+        """push_tokens; with the arguments of the decode that follows, a token
+        that fills no buffer is appended and decoded by one kitty_decode_step
+        call.  True when it was (a spill comes between the two otherwise)."""
+        cfg = self.config
+        S, G = cfg.sink_size, cfg.q_buffer_size
+        ids = tuple(seq_ids)
+        slots = self._slots(ids)
+        if decode is not None:
+            decode.plan_pages = self._longest(layer_id, slots)
         keys = keys.to(self.device, self._dtype)
         values = values.to(self.device, self._dtype)
         l = layer_id
@@ -324,7 +335,8 @@ class KittyInferencePipeline:
         if decode is None:
             _hip.check(self._lib.kitty_append_tokens(ctypes.byref(a), stream))
         else:
-            _hip.check(self._lib.kitty_decode_step(ctypes.byref(a), ctypes.byref(decode), stream))
+            _hip.check(self._lib.kitty_decode_step(ctypes.byref(a), ctypes.byref(decode),
+                                                   self._tickets.data_ptr() + 4 * l * self.num_slots, stream))
 
     def _append_setup(self, l: int, slots: np.ndarray, H: int, D: int) -> Tuple[_hip.AppendArgs, torch.Tensor]:
         """kitty_append_tokens arguments of layer l for these slots, bar the
