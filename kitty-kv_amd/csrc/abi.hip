@@ -27,7 +27,9 @@ static int64_t resident_waves(int waves_per_cu = 8)
 }
 
 // Units the unit-balanced plan charges per 128 sink + tail tokens: the MFMA
-// kernel's FP16 path against one page of the same pair.
+// kernel's FP16 path against one page of the same pair.  3, 4, 5 and 6 took 265,
+// 250, 245 and 242 us where 8 takes 242 (64 ragged sequences to 64K tokens), and
+// 23.9, 23.3, 22.6 and 22.7 against 21.0 (8 x 3-9K, bf16).
 #ifndef KITTY_FP16_WEIGHT_GQ4
 #define KITTY_FP16_WEIGHT_GQ4 8
 #endif

@@ -1314,8 +1314,8 @@ __device__ __forceinline__ DecodeParams kernel_params(KernargParams pp)
 // partial's m is NaN if a key-only page id lies outside the pool.
 // Bound by its chain of loads, MFMAs and softmax per step, not by the units:
 // PV on the VALU (lane = channel pair, fp32 P) and four scores per lane for
-// every group took 15.8 us where this takes 13.5 (1 x 1,024 tokens, pair
-// kernel) and 22.3 against 21.6 (8 x 3-9K tokens, bf16, split).  q is loaded
+// every group took 13.8 us where this takes 12.6 (1 x 1,024 tokens, split and
+// merge) and 24.6 against 23.3 (8 x 3-9K tokens, bf16).  q is loaded
 // again by every step: kept, with 16-bit terms, the split kernel spilled 25-43
 // registers (16 x 32K tokens: 80 us instead of 66), and even 8 spilled ones cost
 // 4 x 128K tokens, groups of 8, 2 us of 76.
@@ -1727,10 +1727,10 @@ void decode_mfma_kernel(DecodeParams p)
 // Such a decode is bound by its chain of launches and dependent loads, not by
 // the chip: a split launch (plan over all sequences, then the first segment),
 // a merge launch, and the append launch before them.  The lengths, q, ranks and
-// page ids are one round trip here.  1 x 512 tokens, 8 KV heads: 11.2 us against
-// 12.0 of the split and merge launches (16.9 with an FP16 walk on the VALU); a
-// module step of 1 x 1,000 tokens 16.0 us against 20.4, of 16 x 1,000 tokens and
-// 8 KV heads 21.3 against 26.0.
+// page ids are one round trip here.  1 x 512 tokens, 8 KV heads: 12.5 us against
+// 12.9 of the split and merge launches, 32 x 512 tokens 15.8 against 21.3; a
+// module step of 1 x 1,000 tokens 16.7 us against 22.6, of 16 x 1,000 tokens and 8
+// KV heads 22.3 against 27.5.
 template <int GQ, bool BF>
 __global__ __launch_bounds__(64 * kPairWaves) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_pair_kernel(DecodeParams p, StepParams step)
