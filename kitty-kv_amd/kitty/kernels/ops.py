@@ -464,16 +464,25 @@ def paged_decode(*args, **kwargs) -> torch.Tensor:
     return decode_plan(*args, **kwargs).run()
 
 
+def calls_followed() -> bool:
+    """True while something records or transforms torch calls rather than run
+    them: torch.jit.trace, torch.compile / export, a dispatch mode (make_fx, fake
+    tensors), forward-mode AD, functorch (vmap, grad).  Some of these hand
+    over plain tensors, and a launch by pointer is invisible to all of them."""
+    return (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
+            or forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
 def plain_rows(*tensors: torch.Tensor) -> bool:
     """True when a kernel may read these (B, heads, T, D) tensors by pointer:
     fp16 or bf16 of one dtype on one ROCm device, with 16-byte aligned rows of contiguous
-    channels.  What a plain launch would drop stays with torch: inputs that
-    need gradients, forward-mode tangents, functorch transforms, tensor
-    subclasses (fake tensors) and negated views."""
+    channels.  What a plain launch would drop stays with torch: calls that
+    are traced or transformed (calls_followed), inputs that need gradients,
+    tensor subclasses and negated views."""
     t0 = tensors[0]
     if t0.device.type != "cuda" or t0.dtype not in (torch.float16, torch.bfloat16):
         return False
-    if forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None:
+    if calls_followed():
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
