@@ -1,6 +1,8 @@
 """Module decode steps whose append and decode go out in one call
 (kitty_decode_step), bit for bit against steps taken apart."""
+import gc
 import warnings
+import weakref
 
 import pytest
 import torch
@@ -96,3 +98,19 @@ def test_full_pool_raises_before_the_step(dev):
     with pytest.raises(RuntimeError, match="exhausted"):
         attn(x(4), x(1), x(1))
     assert torch.equal(pipe.lens, before)
+
+
+@pytest.mark.gpu
+def test_steps_keep_no_plan_alive(dev):
+    """The module keeps at most the 16 plans of _plans (each with a workspace of
+    its own), whatever batches have stepped and whichever were reset since."""
+    layout, pipe, layers = _module("float16", 4, 1, 24, 256)
+    attn = layers[0]
+    x = lambda h: torch.ones(1, h, 1, 128, dtype=torch.float16, device=dev)
+    plans = []
+    for s in range(24):
+        attn(x(4), x(1), x(1), seq_id=s)
+        plans += [weakref.ref(p) for p in attn._plans.values() if p not in [r() for r in plans]]
+        attn(x(4), x(1), x(1), seq_id=s)
+    gc.collect()
+    assert len(plans) == 24 and sum(r() is not None for r in plans) == len(attn._plans) <= 16
