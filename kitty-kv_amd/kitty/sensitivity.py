@@ -226,17 +226,18 @@ class KittySensitivityProfiler:
                 return False
         layers = (_hip.ScoreLayer * n)()
         fresh = [l for l, acc in enumerate(accs) if acc._sum is None]
-        sums = torch.empty(len(fresh), H, D, dtype=torch.float32, device=dev)
-        for l, acc in enumerate(accs):
-            old = acc._sum is not None
-            if not old:
-                acc._sum_abs = sums[fresh.index(l)]
-            layers[l] = _hip.ScoreLayer(acc._slots.data_ptr() if acc._pending else None, acc._sum.data_ptr(),
-                                        float(acc.token_count), int(old))
+        sums = dict(zip(fresh, torch.empty(len(fresh), H, D, dtype=torch.float32, device=dev)))
         both = torch.empty(5 * n * H * D, dtype=torch.uint8, device=dev)     # scores (fp32), then ranks
+        for l, acc in enumerate(accs):
+            layers[l] = _hip.ScoreLayer(acc._slots.data_ptr() if acc._pending else None,
+                                        (sums[l] if l in sums else acc._sum).data_ptr(), float(acc.token_count),
+                                        int(l not in sums))
         _hip.check(_hip.load().kitty_channel_scores(layers, n, H, D, cfg.d_boost, cfg.sentinel, both.data_ptr(),
                                                     both.data_ptr() + 4 * n * H * D, _hip.stream_ptr(dev)))
-        for acc in accs:
+        # the accumulators take the new sums only once the launch that writes them is out
+        for l, acc in enumerate(accs):
+            if l in sums:
+                acc._sum_abs = sums[l]
             acc._pending = False
         host = both.cpu()
         self.scores_ = host[:4 * n * H * D].view(torch.float32).view(n, H, D).clone()

@@ -88,3 +88,28 @@ def test_layers_without_calibration_score_zero(dev):
     with pytest.raises(RuntimeError, match="No tokens"):
         prof.accumulator(2)
         prof.compute()
+
+
+@pytest.mark.gpu
+def test_failed_scores_leave_the_sums(dev, monkeypatch):
+    """A compute() whose launch is refused raises and loses nothing."""
+    from kitty import _hip
+    cfg = _cfg(2, 1, 128)
+    prof = KittySensitivityProfiler(cfg)
+    keys = [torch.randn(1, 1, 64, 128).half() for _ in range(2)]
+    for l in range(2):
+        prof.update(l, keys[l].to(dev))
+
+    class Refusing:
+        def __getattr__(self, name):
+            return (lambda *a: _hip.KITTY_E_HIP) if name == "kitty_channel_scores" else getattr(real, name)
+    real = _hip.load()
+    with monkeypatch.context() as m:
+        m.setattr(_hip, "_lib", Refusing())
+        with pytest.raises(RuntimeError):
+            prof.compute()
+    for l in range(2):
+        want = keys[l].double().abs().sum((0, 2))
+        assert torch.allclose(prof.accumulator(l).sum_abs.cpu().double(), want, rtol=1e-5)
+    prof.compute()
+    assert torch.allclose(prof.scores_[1, 0].double(), keys[1].double().abs().mean((0, 1, 2)), rtol=1e-5)
