@@ -372,14 +372,26 @@ struct WaveState {
 // scaled by 4^a, zero-point term Y not yet subtracted).
 //  P' = p * s_t (value scale of token t) is written to LDS as three fp8
 //  terms on MFMA rows 4h + t: term 0 = fp8(P' / sig), term t encodes the
-//  remaining residual with scale sig / 16^t (about 12 significant bits in
-//  all).  sig = 2^(e - 8) with s_max < 2^e, the page's largest value scale,
-//  so P' / sig < 256 <= 448 (p <= 1).
+//  remaining residual with scale sig / 64^t (12 significant bits in all, or
+//  2^-24 of s_max).  sig = 2^(e - 4) with s_max < 2^e, the page's largest value
+//  scale, so P' / sig < 16 (p <= 1), and the residuals stay below 64 of their
+//  scales (fp8 ends at 448).
+//  The matrix core aligns a row's products to the largest and drops what lies
+//  below its window, so a term 0 that spans fp8's range loses the low bits of
+//  all but a page's top tokens, the more the more pages start a chunk (p = 1 in
+//  each).  Below 2^-6 fp8 is fixed-point, whose sums lose nothing; what a smaller
+//  term 0 leaves is the other terms', which need the wide step for it.  Error
+//  against float64, 1 x 1,024 tokens of 8 heads / 1 x 30,000 of 32 / 16 x 32K / 1 x
+//  30,000 in chunks of 64 pages: sig 2^(e - 8), steps of 16, 4.6e-4 / 9.5e-4 / 6.8e-4 /
+//  6.3e-4; 2^(e - 4), 16: 2.14e-4 / 2.10e-4 / 2.57e-4 / 5.2e-4; 2^(e - 4), 64: 2.14e-4 /
+//  2.07e-4 / 2.02e-4 / 2.08e-4, the rounding of the output.
 //  Value codes: two tr4 reads per 8-byte chunk ch give each lane the nibble
 //  of channels 32ch + 2r, +1 for tokens 32q + 0..31; the nibble masked with
 //  0x3 (even channel) or shifted down by 2 (odd) is the fp4 operand.
-//  O[h][d] += 2 sig (C0 + C1 / 16 + C2 / 256) - sum_t P'_t z_t, C_t = row
+//  O[h][d] += 2 sig (C0 + C1 / 64 + C2 / 64^2) - sum_t P'_t z_t, C_t = row
 //  4h + t of the MFMA output (fp4 value = code / 2).
+constexpr float kTermStep = 1.0f / 64.0f;
+
 template <int GQ>
 __device__ __forceinline__ void pv_fp8_fp4(WaveState<GQ, false> &W, unsigned char *st, const f32x4 (&S)[2][4],
                                            const f32x4 &Yt, int lane)
@@ -433,7 +445,7 @@ __device__ __forceinline__ void pv_fp8_fp4(WaveState<GQ, false> &W, unsigned cha
     W.l_run[0] = W.l_run[0] * alpha + lsum;
     const float yv = row_sum16(ysum);
     smax = row_max16(smax);
-    const float sig = __builtin_amdgcn_ldexpf(1.0f, __builtin_amdgcn_frexp_expf(smax) - 8);
+    const float sig = __builtin_amdgcn_ldexpf(1.0f, __builtin_amdgcn_frexp_expf(smax) - 4);
 
     unsigned char *pb = st + kKlo;  // 16 rows x 128 fp8, over the consumed key codes
 #pragma unroll
@@ -441,9 +453,9 @@ __device__ __forceinline__ void pv_fp8_fp4(WaveState<GQ, false> &W, unsigned cha
         float *xc = x[cb];
         unsigned w0 = fp8x4(xc[0], xc[1], xc[2], xc[3], sig);
         fp8_residual(xc, w0, sig);
-        unsigned w1 = fp8x4(xc[0], xc[1], xc[2], xc[3], sig * 0.0625f);
-        fp8_residual(xc, w1, sig * 0.0625f);
-        unsigned w2 = fp8x4(xc[0], xc[1], xc[2], xc[3], sig * 0.00390625f);
+        unsigned w1 = fp8x4(xc[0], xc[1], xc[2], xc[3], sig * kTermStep);
+        fp8_residual(xc, w1, sig * kTermStep);
+        unsigned w2 = fp8x4(xc[0], xc[1], xc[2], xc[3], sig * (kTermStep * kTermStep));
         unsigned char *row = pb + 128 * (4 * q) + 64 * cb + 4 * r;
         *(unsigned *)(row) = w0;
         *(unsigned *)(row + 128) = w1;
@@ -476,8 +488,8 @@ __device__ __forceinline__ void pv_fp8_fp4(WaveState<GQ, false> &W, unsigned cha
                           ((unsigned)vr[ch][1][0] >> 2) & m, ((unsigned)vr[ch][1][1] >> 2) & m};
         const f32x4 ce = mfma_fp8_fp4(Ap, ev);
         const f32x4 co = mfma_fp8_fp4(Ap, od);
-        const float ve = __builtin_fmaf(ce[2], 0.00390625f, __builtin_fmaf(ce[1], 0.0625f, ce[0]));
-        const float vo = __builtin_fmaf(co[2], 0.00390625f, __builtin_fmaf(co[1], 0.0625f, co[0]));
+        const float ve = __builtin_fmaf(ce[2], kTermStep * kTermStep, __builtin_fmaf(ce[1], kTermStep, ce[0]));
+        const float vo = __builtin_fmaf(co[2], kTermStep * kTermStep, __builtin_fmaf(co[1], kTermStep, co[0]));
         W.o4[ch][0] = __builtin_fmaf(W.o4[ch][0], alpha, __builtin_fmaf(ve, s2, -yv));
         W.o4[ch][1] = __builtin_fmaf(W.o4[ch][1], alpha, __builtin_fmaf(vo, s2, -yv));
     }

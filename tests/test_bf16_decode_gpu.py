@@ -13,12 +13,12 @@ from kvgen import calibrate_boost_idx, outlier_keys
 G = D = 128
 
 
-def _case(dev, seed, Hq, H, Dk, pages_k, pages_v, tails, sinks, key_scale=1.0, val_scale=1.0, q_scale=1.0):
-    """Pools quantised on the device from bf16 blocks and the decode operands;
+def _case(dev, seed, Hq, H, Dk, pages_k, pages_v, tails, sinks, key_scale=1.0, val_scale=1.0, q_scale=1.0,
+          bf=torch.bfloat16):
+    """Pools quantised on the device from bf16 (or fp16) blocks and the decode operands;
     pages_v None: one stream."""
     from kitty.kernels.ops import pool_store, quantize_into_pools
     gen = torch.Generator().manual_seed(seed)
-    bf = torch.bfloat16
     B, n = len(pages_k), sum(pages_k)
     K, chans = outlier_keys(gen, (max(n, 1) * G,), H, D, max(Dk, 1), 8.0)
     K = (K.float() * key_scale).to(bf).to(dev)
