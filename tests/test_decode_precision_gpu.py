@@ -21,3 +21,16 @@ def test_fp16_decode_error(dev, Hq, H, Dk, pages, tails, per_split):
     # both round the output to fp16, about 2.1e-4 of it; what the fp8 terms
     # add (12 bits each, 1e-5 of the output over a page) is not to show in it
     assert e_fast <= 1.05 * e_gen + 1e-6, (e_fast, e_gen)
+
+
+# sharp to flat softmax rows: the flatter, the more the zero points cancel
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1.0, 0.5, 0.2])
+@pytest.mark.parametrize("Hq,H,Dk,pages", [(32, 8, 16, [200]), (16, 4, 32, [90, 3]), (64, 8, 16, [160]), (32, 2, 0, [120])])
+def test_bf16_decode_error(dev, Hq, H, Dk, pages, scale):
+    args, kw = _case(dev, 3 * Hq + len(pages), Hq, H, Dk, pages, None, [20] * len(pages), [32] * len(pages), q_scale=scale)
+    ref = _float64(args, kw)
+    fast, gen = _run(args, kw, boost_unique=True), _run(args, kw, boost_unique=False)
+    e_fast, e_gen = (float((x - ref).norm() / ref.norm()) for x in (fast, gen))
+    # an error of up to 1e-5 of the output, in quadrature with its fp16 rounding of 2.1e-4
+    assert e_fast <= 1.001 * e_gen + 1e-7, (e_fast, e_gen)
