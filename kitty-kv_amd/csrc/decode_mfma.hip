@@ -513,8 +513,10 @@ __device__ __forceinline__ void pv_fp8_fp4(WaveState<GQ, false> &W, unsigned cha
 // where they are read, each of the 16 lanes of a group would redo its
 // 40 words: 120 VALU against 12).  q enters times 2^9 (qk_setup), so that the
 // products and their residuals stay clear of fp16's subnormals.  A page
-// with a scale of 16 or more is brought below it by a power of two, 1 / kmul,
-// which the scores take back, so any bf16 scale decodes.
+// whose largest scale is 16 or more, or below 2^-6, is brought to [8, 16) by a
+// power of two, 1 / kmul, which the scores take back: scales decode with all
+// their bits down to 2^-12 of 2^-6 or of the page's largest (fp16 subnormals
+// below).
 template <int GQ, bool BF>
 __device__ __forceinline__ void page_qk(const WaveState<GQ, BF> &W, unsigned char *st, int lane, int Dk,
                                         f32x4 (&S)[2][4], f32x4 &Yt, float &kmul)
@@ -536,11 +538,12 @@ __device__ __forceinline__ void page_qk(const WaveState<GQ, BF> &W, unsigned cha
         }
         const unsigned mag = max(max(w0 << 16 & 0x7fffffffu, w0 & 0x7fff0000u), max(w1 << 16 & 0x7fffffffu, w1 & 0x7fff0000u));
         float f0 = bf_lo(w0), f1 = bf_hi(w0), f2 = bf_lo(w1), f3 = bf_hi(w1);
-        if (__builtin_expect(__ballot(lane < 32 && mag >= 0x41800000u) != 0, 0)) {
+        const uint64_t big = __ballot(lane < 32 && mag >= 0x41800000u), mid = __ballot(lane < 32 && mag >= 0x3c800000u);
+        if (__builtin_expect(big != 0 || mid == 0, 0)) {
             int e = lane < 32 ? (int)(mag >> 23) : 0;   // biased exponent
             for (int off = 1; off < 64; off <<= 1)
                 e = max(e, __shfl_xor(e, off));
-            const int k = e - 130;                      // the largest scale below 2^4
+            const int k = max(e - 130, -126);           // the largest scale in [2^3, 2^4)
             kmul = __builtin_amdgcn_ldexpf(1.0f, k);
             if (lane < 32) {
                 f0 = __builtin_amdgcn_ldexpf(f0, -k), f1 = __builtin_amdgcn_ldexpf(f1, -k);

@@ -34,3 +34,21 @@ def test_bf16_decode_error(dev, Hq, H, Dk, pages, scale):
     e_fast, e_gen = (float((x - ref).norm() / ref.norm()) for x in (fast, gen))
     # an error of up to 1e-5 of the output, in quadrature with its fp16 rounding of 2.1e-4
     assert e_fast <= 1.001 * e_gen + 1e-7, (e_fast, e_gen)
+
+
+# key scales that fp16 holds in few bits or not at all, with queries that make
+# their scores count; value scales down to 2^-114
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq", [4, 8, 16])
+@pytest.mark.parametrize("key_exp,val_exp", [(-20, 0), (-34, -20), (-60, 0), (-100, 0), (0, -114)])
+def test_bf16_tiny_scales(dev, Hq, key_exp, val_exp):
+    args, kw = _case(dev, 37, Hq, 1, 16, [5], [4], [9], [32], q_scale=2.0 ** min(-key_exp, 100))
+    q, sk, tk, km, vm = args[0], args[9], args[12], args[5], args[7]
+    km[:, :, 0] *= 2.0 ** key_exp
+    vm[:, :, :, 0] *= 2.0 ** val_exp
+    sk *= 2.0 ** key_exp
+    tk *= 2.0 ** key_exp
+    ref = _float64(args, kw)
+    fast, gen = _run(args, kw, boost_unique=True), _run(args, kw, boost_unique=False)
+    e_fast, e_gen = (float((x - ref).norm() / ref.norm()) for x in (fast, gen))
+    assert e_fast <= 1.05 * e_gen + 1e-6, (e_fast, e_gen)
