@@ -635,6 +635,10 @@ bool page128_supported(const kitty_page_store &st, const kitty_quant_batch &qb)
 {
     if (st.head_dim != 128 || st.page_tokens != 128)
         return false;
+    // fp16 blocks take the packed fp16 instance, which needs finite elements: into
+    // bf16 pools they keep the shape-generic kernel, whose ranges skip NaN elements
+    if (qb.src_dtype == KITTY_DTYPE_F16 && st.meta_dtype != KITTY_DTYPE_F16)
+        return false;
     if (qb.key) {
         // token-major rows (channel stride 1) or channel-major rows (token stride 1)
         const bool rows = qb.key_s_chan == 1 && mul(qb.key_s_tok, 8);

@@ -119,3 +119,23 @@ def test_bf16_value_shift(dev):
                         value_shift=R)
     plan.run()
     assert torch.equal(buf[:, :, :R], before[:, :, G:]) and torch.equal(buf[:, :, R:], before[:, :, R:])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["normal", "ties", "constant", "nonfinite"])
+def test_fp16_blocks_into_bf16_pools(dev, kind):
+    """fp16 blocks into bf16 pools quantise as on the shape-generic kernel
+    whatever their alignment, all-NaN channels and tokens included."""
+    from kitty.kernels.ops import pool_store, quantize_into_pools
+    gen = torch.Generator().manual_seed(60 + KINDS.index(kind))
+    n, H, Dk = 2, 2, 16
+    k, v = (_blocks(kind, n, H, gen).to(torch.float16).to(dev) for _ in range(2))
+    bi = torch.full((H, D), Dk + 1, dtype=torch.uint8, device=dev)
+    bi[:, :Dk] = torch.arange(Dk, dtype=torch.uint8, device=dev)
+    ids = torch.tensor([1, 0], dtype=torch.int32, device=dev)
+    got, ref = _pools(n, H, Dk, torch.bfloat16, dev), _pools(n, H, Dk, torch.bfloat16, dev)
+    quantize_into_pools(pool_store(*got), k, v, bi, ids, Dk + 1)
+    quantize_into_pools(pool_store(*ref), _misaligned(k), _misaligned(v), bi, ids, Dk + 1)
+    for a, b in zip(got, ref):
+        a, b = (t.view(torch.int16) if t.element_size() == 2 else t for t in (a, b))
+        assert torch.equal(a, b)
