@@ -362,9 +362,10 @@ int kitty_decode_step(const kitty_append_args *append, const kitty_decode_args *
  * aligned with strides that are multiples of 4; token strides of k and v
  * non-negative with a head's rows inside 2 GiB; other layouts return
  * KITTY_E_UNSUPPORTED.  Scores that are NaN or +infinity give NaN rows, as
- * the softmax does; a NaN or infinite value row j may also reach rows
- * i < j of the same 64-token tile (their weight 0 times it), and an infinite
- * value gives NaN where the plain product would give infinity. */
+ * the softmax does; a NaN or infinite value reaches the rows that weigh it
+ * as the product with their weights does, and may reach rows i < j of its
+ * 64-token tile as NaN (weight 0 times it).  bf16 values are to stay below
+ * 2^100 (the products are summed times up to 2^15). */
 typedef struct {
     const uint16_t *q, *k, *v; /* (B, Hq, T, D), (B, Hkv, T, D) twice */
     uint16_t *out;             /* (B, Hq, T, D) */

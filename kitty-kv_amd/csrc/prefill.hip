@@ -279,21 +279,59 @@ void prefill_attention_kernel(PrefillParams p)
             tile_step<BF16>(W, k1, v1, (t + 1) * kTile, p.c, g);
     }
 
-    const float inv = 1.0f / other_sum(W.l);
-    if (active && W.q_lo + n < p.T) {
-        uint16_t *o = p.out + b * p.o_s_seq + h * p.o_s_head + W.qi * p.o_s_tok;
+    const float lsum = other_sum(W.l), inv = 1.0f / lsum;
+    const bool row = active && W.q_lo + n < p.T;
+    uint16_t *o = p.out + b * p.o_s_seq + h * p.o_s_head + W.qi * p.o_s_tok;
+    bool odd = false;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint16_t r[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                r[e] = f2x(W.O[dt][4 * j + e] * inv, BF16);
+                odd |= !(__builtin_fabsf(W.O[dt][4 * j + e]) < __builtin_inff());
+            }
+            if (row)
+                *(uint2 *)(o + 32 * dt + 8 * j + 4 * g) =
+                    make_uint2((uint32_t)r[0] | ((uint32_t)r[1] << 16), (uint32_t)r[2] | ((uint32_t)r[3] << 16));
+        }
+
+    // Infinite values: the second term of a weight is 0 or negative where the
+    // weight is not, and times infinity makes the sum NaN (as does the weight 0
+    // of a later token in the tile).  A wave that met one sums the infinities and
+    // NaNs of the value rows its queries see, and writes those sums; rows whose
+    // softmax is itself NaN stay as they are.
+    odd = odd && row && lsum > 0.0f && lsum < __builtin_inff();
+    if (!__ballot(odd))
+        return;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            W.O[dt][i] = 0.0f;
+    for (int t = 0; t <= min(W.q_lo + kRows, p.T) - 1; ++t) {
+        const unsigned char *vrow = vp + (uint32_t)t * p.v_row + 8 * g;
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                uint16_t r[4];
+                const uint2 v = *(const uint2 *)(vrow + 64 * dt + 16 * j);
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    r[e] = f2x(W.O[dt][4 * j + e] * inv, BF16);
-                *(uint2 *)(o + 32 * dt + 8 * j + 4 * g) =
-                    make_uint2((uint32_t)r[0] | ((uint32_t)r[1] << 16), (uint32_t)r[2] | ((uint32_t)r[3] << 16));
+                for (int e = 0; e < 4; ++e) {
+                    const float x = x2f((uint16_t)((e < 2 ? v.x : v.y) >> (16 * (e & 1))), BF16);
+                    if (t <= W.qi && !(__builtin_fabsf(x) < __builtin_inff()))
+                        W.O[dt][4 * j + e] += x;
+                }
             }
     }
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (odd && !(__builtin_fabsf(W.O[dt][i]) < __builtin_inff()))
+                o[32 * dt + 8 * (i >> 2) + 4 * g + (i & 3)] = f2x(W.O[dt][i], BF16);
 }
 
 static bool al(const void *p, unsigned a) { return ((uintptr_t)p & (a - 1)) == 0; }

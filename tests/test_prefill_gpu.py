@@ -91,6 +91,40 @@ def test_prefill_nonfinite_rows(dev):
             assert out[i].isfinite().all(), i
 
 
+# one head and groups; an infinite value at the first token (weight 1 in its own
+# row), inside tiles, of both signs in one channel, in the last ragged tile
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,T,rows", [(1, 1, 1, [(0, 5, 1)]), (4, 1, 40, [(0, 3, 1), (7, 3, -1), (9, 4, -1)]),
+                                           (6, 2, 201, [(0, 0, -1), (70, 5, 1), (75, 6, -1), (150, 5, -1), (200, 7, 1)])])
+def test_prefill_nonfinite_values(dev, dtype, Hq, Hkv, T, rows):
+    """Infinite and NaN values reach the rows that see them as the product of the
+    weights with them does; other channels and tiles before keep their numbers."""
+    from kitty.kernels.ops import prefill_attention
+    gen = torch.Generator().manual_seed(T)
+    q, k, v = (torch.randn(1, h, T, 128, generator=gen).to(dtype) for h in (Hq, Hkv, Hkv))
+    clean = _ref(q, k, v)
+    for t, c, sign in rows:
+        v[0, :, t, c] = sign * float("inf")
+    v[0, :, T // 2, 100] = float("nan")
+    out = prefill_attention(q.to(dev), k.to(dev), v.to(dev), 1.0 / math.sqrt(128)).cpu().double()
+    bad = {c for _, c, _ in rows} | {100}
+    keep = [c for c in range(128) if c not in bad]
+    eps = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    assert ((out - clean).abs() <= eps * clean.abs() + 1e-4)[..., keep].all()
+    for h in range(Hq):
+        s = (q[0, h].double() @ k[0, h * Hkv // Hq].double().t()) / math.sqrt(128)
+        for i in range(T):
+            want = torch.softmax(s[i, :i + 1], 0) @ v[0, h * Hkv // Hq, :i + 1].double()
+            for c in bad:
+                first = min([t for t, cc, _ in rows if cc == c] + [T // 2] * (c == 100))
+                if i >= first:
+                    got = out[0, h, i, c]
+                    assert got == want[c] or (got.isnan() and want[c].isnan()), (h, i, c)
+                elif i // 64 < first // 64:
+                    assert (out[0, h, i, c] - clean[0, h, i, c]).abs() <= eps * clean[0, h, i, c].abs() + 1e-4
+
+
 @pytest.mark.gpu
 def test_module_prefill_keeps_gradients(dev):
     """Inputs that need gradients keep torch's differentiable path."""
