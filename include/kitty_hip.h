@@ -347,8 +347,12 @@ int kitty_append_tokens(const kitty_append_args *args, kitty_stream_t stream);
  * call (kitty/attention.py:74-151, ABI version 7).  The decode's arguments are
  * checked before anything is launched.  With tickets (device, an int32 per slot
  * of the append, all 0; each call leaves them 0) a batch of few pairs and pages
- * takes one launch, for which the decode's buffers and lengths have to be those
- * the append writes (decode->sink_len[b] == append->sink_fill[slots[b]] and so on). */
+ * takes one launch where the decode reads the append's own buffers and counters
+ * for a run of slots (decode->sink_len == append->sink_fill + s, decode->tail_k.ptr
+ * == append->buf_k + s * s_slot and so on, and slots[b] == s + b on the device: a
+ * sequence whose slot is another one is not appended and has overflow[b] set);
+ * any other arguments take the separate launches.  A launch that is lost half-way
+ * leaves tickets behind: zero them with the buffers it wrote. */
 int kitty_decode_step(const kitty_append_args *append, const kitty_decode_args *decode, int32_t *tickets,
                       kitty_stream_t stream);
 

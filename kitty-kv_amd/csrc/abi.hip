@@ -388,12 +388,30 @@ extern "C" int kitty_paged_decode(const kitty_decode_args *args, kitty_stream_t 
     return rc || p.B == 0 ? rc : launch_decode(p, args, stream);
 }
 
-// The append's buffers are the decode's, as far as the pair kernel relies on it.
-static bool step_fits(const kitty_append_args &a, const kitty_decode_args &d)
+// The append's first slot if the decode reads the append's own buffers and
+// counters, from that slot on in a run of d.batch; else -1 (such a step takes two
+// launches: in one, rows would land where the decode's lengths say).
+static int step_slot0(const kitty_append_args &a, const kitty_decode_args &d)
 {
-    return a.batch == d.batch && a.num_kv_heads == d.num_kv_heads && a.head_dim == d.head_dim &&
-           (a.val_len != nullptr) == (d.tail_len_v != nullptr) && a.sink_size == d.sink_capacity &&
-           a.buf_tokens == d.tail_capacity && (!a.val_len || a.val_tokens == d.tail_v_capacity);
+    if (a.batch != d.batch || a.num_kv_heads != d.num_kv_heads || a.head_dim != d.head_dim ||
+        (a.val_len != nullptr) != (d.tail_len_v != nullptr) || a.sink_size != d.sink_capacity ||
+        a.buf_tokens != d.tail_capacity || (a.val_len && a.val_tokens != d.tail_v_capacity))
+        return -1;
+    const int64_t off = (int64_t)((uintptr_t)d.sink_len - (uintptr_t)a.sink_fill);
+    const int64_t s0 = off / (int64_t)sizeof(int32_t);
+    if (off % (int64_t)sizeof(int32_t) || s0 < 0 || s0 + a.batch > a.num_slots || d.tail_len != a.buf_len + s0 ||
+        (a.val_len && d.tail_len_v != a.val_len + s0))
+        return -1;
+    auto same = [&](const kitty_fp16_seg &seg, const uint16_t *buf, const kitty_slot_layout &l) {
+        return seg.ptr == buf + s0 * l.s_slot && seg.s_tok == l.s_tok && (a.num_kv_heads == 1 || seg.s_head == l.s_head) &&
+               (a.batch == 1 || seg.s_seq == l.s_slot);
+    };
+    if (a.sink_size > 0 && (!same(d.sink_k, a.sink_k, a.sink_layout) || !same(d.sink_v, a.sink_v, a.sink_layout)))
+        return -1;
+    if (!same(d.tail_k, a.buf_k, a.buf_layout) ||
+        !(a.val_len ? same(d.tail_v, a.val_buf, a.val_layout) : same(d.tail_v, a.buf_v, a.buf_layout)))
+        return -1;
+    return (int)s0;
 }
 
 extern "C" int kitty_decode_step(const kitty_append_args *append, const kitty_decode_args *decode, int32_t *tickets,
@@ -403,11 +421,13 @@ extern "C" int kitty_decode_step(const kitty_append_args *append, const kitty_de
     int rc = prepare(decode, p);
     if (rc)
         return rc;
-    if (append && tickets && p.B > 0 && p.sub_groups == 1 && p.pair && step_fits(*append, *decode)) {
+    if (append && tickets && p.B > 0 && p.sub_groups == 1 && p.pair) {
         rc = check_append(append);
         if (rc)
             return rc;
-        return launch_pair(p, StepParams{*append, tickets}, (hipStream_t)stream);
+        const int slot0 = step_slot0(*append, *decode);
+        if (slot0 >= 0)
+            return launch_pair(p, StepParams{*append, tickets, slot0}, (hipStream_t)stream);
     }
     rc = kitty_append_tokens(append, stream);
     return rc || p.B == 0 ? rc : launch_decode(p, decode, stream);

@@ -193,10 +193,12 @@ __host__ __device__ inline int xcd_local_index(int i, int n)
 constexpr int kPairWaves = 8;
 
 // The append of a decode step in the pair kernel's launch; tickets NULL: no
-// append.  tickets: an int32 per slot, 0 between launches.
+// append.  tickets: an int32 per slot, 0 between launches.  The decode's rows
+// and lengths are those of the append's slots slot0, slot0 + 1, ...
 struct StepParams {
     kitty_append_args append;
     int32_t *tickets;
+    int slot0;
 };
 
 size_t generic_lds_bytes(int GQ, int D, int G, int Dk);

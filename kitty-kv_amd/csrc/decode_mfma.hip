@@ -1775,8 +1775,7 @@ void decode_pair_kernel(DecodeParams p, StepParams step)
         const kitty_append_args &a = step.append;
         slot = a.slots[b];
         to_sink = ns < a.sink_size;
-        fresh = slot >= 0 && slot < a.num_slots &&
-                (to_sink || !(nk >= a.buf_tokens || (a.val_len && nv >= a.val_tokens)));
+        fresh = slot == step.slot0 + b && (to_sink || !(nk >= a.buf_tokens || (a.val_len && nv >= a.val_tokens)));
     }
     const int ns0 = ns, nk0 = nk, nv0 = nv;
     if (fresh) {
@@ -1834,10 +1833,10 @@ void decode_pair_kernel(DecodeParams p, StepParams step)
     if (step.tickets && threadIdx.x == 0) {
         const kitty_append_args &a = step.append;
         // the last of the sequence's Hkv workgroups; the ticket wraps to 0 with it
-        if (slot >= 0 && slot < a.num_slots &&
-            atomicInc((unsigned *)step.tickets + slot, (unsigned)p.Hkv - 1) == (unsigned)p.Hkv - 1) {
-            if (!fresh) {
-                a.overflow[b] = 1;
+        if (atomicInc((unsigned *)step.tickets + step.slot0 + b, (unsigned)p.Hkv - 1) == (unsigned)p.Hkv - 1) {
+            if (!fresh) {   // a full buffer, or a slot that is not the row the decode reads
+                if (slot >= 0 && slot < a.num_slots)
+                    a.overflow[b] = 1;
             } else if (to_sink) {
                 a.sink_fill[slot] = ns0 + 1;
             } else {

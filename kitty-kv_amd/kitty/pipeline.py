@@ -878,6 +878,7 @@ class KittyInferencePipeline:
                    for t in (self._sink_k, self._sink_v, self._qbuf_k, self._vbuf)]
         regions.append(_hip.ZeroRegion(self._block_table.data_ptr() + 4 * s * maxp, L, 4 * maxp, 4 * n * maxp))
         regions.append(_hip.ZeroRegion(self.lens.data_ptr() + 4 * s, 5 * L, 4, 4 * n))
+        regions.append(_hip.ZeroRegion(self._tickets.data_ptr() + 4 * s, L, 4, 4 * n))
         return (_hip.ZeroRegion * len(regions))(*regions)
 
     def stats(self) -> dict:

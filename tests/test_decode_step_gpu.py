@@ -1,9 +1,11 @@
 """Module decode steps whose append and decode go out in one call
 (kitty_decode_step), bit for bit against steps taken apart."""
+import ctypes
 import gc
 import warnings
 import weakref
 
+import numpy as np
 import pytest
 import torch
 
@@ -114,3 +116,73 @@ def test_steps_keep_no_plan_alive(dev):
         attn(x(4), x(1), x(1), seq_id=s)
     gc.collect()
     assert len(plans) == 24 and sum(r() is not None for r in plans) == len(attn._plans) <= 16
+
+
+def _raw_step(dev, B, slots):
+    """A pipeline of four 100-token sequences and the arguments of a step of the
+    decode's rows 1 .. B with the append's slots."""
+    from kitty import _hip
+    layout, pipe, layers = _module("float16", 8, 2, 4, 512)
+    gen = torch.Generator().manual_seed(8)
+    k = torch.randn(4, 2, 100, 128, generator=gen).half().to(dev)
+    pipe.push_chunk(0, k, -k, [0, 1, 2, 3])
+    tok = torch.randn(B, 2, 128, generator=gen).half().to(dev)
+    q = torch.randn(B, 8, 1, 128, generator=gen).half().to(dev)
+    plan = layers[0]._plan(q[:, :, 0].contiguous(), list(range(1, 1 + B)))
+    a, keep = pipe._append_setup(0, np.array(slots), 2, 128)
+    a.key = a.value = tok.data_ptr()
+    a.key_s_seq = a.value_s_seq = 256
+    a.key_s_head = a.value_s_head = 128
+    out = torch.empty_like(q)
+    d = plan.step_args(q, out)
+    d.plan_pages = 1
+
+    def step():
+        _hip.check(pipe._lib.kitty_decode_step(ctypes.byref(a), ctypes.byref(d), pipe._tickets.data_ptr(),
+                                               _hip.stream_ptr(dev)))
+        torch.cuda.synchronize()
+    return pipe, d, tok, out, step, (layers, plan, q, keep)
+
+
+@pytest.mark.gpu
+def test_step_whose_lengths_are_not_the_appends(dev):
+    """A decode over a copy of the counters: the token goes where the append's
+    own counters say, the decode sees the lengths it was given."""
+    pipe, d, tok, out, step, _keep = _raw_step(dev, 2, [1, 2])
+    lens = pipe.lens[:, 0, 1:3].clone()
+    lens[1] -= 5
+    lens[4] -= 5                                   # five tokens fewer: rows 63 .. 67 are not theirs
+    d.sink_len, d.tail_len, d.num_pages, d.num_pages_v, d.tail_len_v = (lens[i].data_ptr() for i in (0, 1, 2, 3, 4))
+    qbuf, vbuf, n = pipe._qbuf_k.clone(), pipe._vbuf.clone(), pipe.lens.clone()
+    step()
+    for s in (1, 2):
+        qbuf[s, 0, :, 68] = tok[s - 1]
+        vbuf[s, 0, :, 68] = tok[s - 1]
+        n[1, 0, s] += 1
+        n[4, 0, s] += 1
+    assert torch.equal(pipe._qbuf_k, qbuf) and torch.equal(pipe._vbuf, vbuf) and torch.equal(pipe.lens, n)
+    assert out.isfinite().all() and not pipe._tickets.any()
+
+
+@pytest.mark.gpu
+def test_step_with_slots_of_other_rows(dev):
+    """Slots that are not the decode's rows are refused, one by one."""
+    pipe, d, tok, out, step, _keep = _raw_step(dev, 3, [1, 3, 2])
+    qbuf, vbuf, n = pipe._qbuf_k.clone(), pipe._vbuf.clone(), pipe.lens.clone()
+    step()
+    qbuf[1, 0, :, 68] = tok[0]
+    vbuf[1, 0, :, 68] = tok[0]
+    n[1, 0, 1] += 1
+    n[4, 0, 1] += 1
+    assert torch.equal(pipe._qbuf_k, qbuf) and torch.equal(pipe._vbuf, vbuf) and torch.equal(pipe.lens, n)
+    assert pipe._overflow.tolist()[:3] == [0, 1, 1] and not pipe._tickets.any()
+
+
+@pytest.mark.gpu
+def test_reset_clears_the_tickets(dev):
+    layout, pipe, layers = _module("float16", 8, 2, 2, 512)
+    x = lambda h: torch.ones(2, h, 1, 128, dtype=torch.float16, device=dev)
+    layers[0](x(8), x(2), x(2))
+    pipe._tickets += 1                              # as a lost launch leaves them
+    pipe.reset_sequence(1)
+    assert pipe._tickets.tolist() == [[1, 0]]
