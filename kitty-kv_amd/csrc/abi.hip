@@ -101,16 +101,32 @@ static void set_plan(DecodeParams &p, const kitty_decode_args &a, bool balanced)
 // and CU, so up to resident_waves(1) pairs, of few units (pages + FP16 units)
 // each.  It saves the merge launch (and a step's append launch), and loses where
 // its 8 waves per pair leave the chip idle that the split plan fills.  Measured
-// in us, one kernel against the two, pages + 18 FP16 units:
-//   8 pairs,   20 units 12.5 / 12.9,  28 units 15.6 / 13.2
-//   64 pairs,  25 units 13.9 / 15.1,  28 units 16.5 / 15.5
-//   128 pairs, 40 units 21.1 / 21.5,  68 units 29.5 / 25.3
-//   256 pairs, 40 units 23.3 / 28.7,  68 units 34.3 / 39.9
-// and a module step (plan_pages given; host-bound up to 16 us) 16.7 / 22.6 with 8
-// pairs of 26 units, 19.2 / 22.6 of 41, 21.5 / 22.9 of 49.  A batch's units are its
-// longest sequence's, and only the split plan evens ragged ones out: at most 48.
+// in us, one kernel against the two, pages + 18 FP16 units, groups of 4 in fp16 |
+// of 8 in bf16:
+//   8 pairs,   20 units 13.1 / 13.8 | 15.3 / 15.2,  25 units 13.6 / 13.6 | 15.9 / 14.5
+//   32 pairs,  20 units 13.5 / 14.4 | 15.8 / 15.5 (groups of 8 in fp16 15.1 / 15.1)
+//   64 pairs,  22 units 13.7 / 15.0 | 15.8 / 16.4,  25 units 14.2 / 14.9 | 16.5 / 16.4
+//   128 pairs, 38 units 19.0 / 22.5 | 24.4 / 26.8,  48 units 21.3 / 23.6 | 29.7 / 28.8
+//   256 pairs, 38 units 20.5 / 26.2 | 26.6 / 33.6,  48 units 23.1 / 28.2 | 31.3 / 38.3
+// A batch's units are its longest sequence's, and only the split plan evens ragged
+// ones out: at most 48.  A module step (plan_pages given) is bound by the host
+// where it takes the separate launches, 21 us with one sequence and 27 with more,
+// and the kernel may take as long (the same two columns, 43 units unless said):
+//   1 sequence,  34 units 16.7 / 20.9 | 19.7 / 21.2,  38 units 18.0 / 20.9 | 22.0 / 21.0,
+//                19.2 / 20.9 | 24.3 / 20.9; groups of 8 in fp16 38 units 19.7 / 20.9, 21.5 / 20.8;
+//                groups of 4 in bf16 34 units 19.2 / 21.1, 38 units 21.2 / 21.0
+//   2 sequences  21.6 / 26.9 | 24.8 / 27.0,   8 sequences 22.0 / 27.3 | 25.6 / 27.3
+//   16 sequences 22.3 / 27.6 | 26.4 / 29.9;   48 units, 2 sequences 21.7 / 26.8 | 28.7 / 27.0
 // A group of 16 heads (4 waves per CU: 20.8 us against 15.3) stays split.
 constexpr int kPairUnits = 21, kPairStepUnits = 44, kPairUnitsMax = 48;
+
+// Units up to which few pairs take the kernel, of a plain decode and of a module step.
+static int pair_units(const DecodeParams &p, bool step)
+{
+    if (!step)
+        return p.act_bf16 && p.GQ > 4 ? 0 : kPairUnits;
+    return p.B > 1 ? kPairStepUnits : (p.act_bf16 ? 34 : (p.GQ > 4 ? 38 : kPairStepUnits));
+}
 
 static bool pair_plan(const DecodeParams &p, const kitty_decode_args &a)
 {
@@ -119,7 +135,7 @@ static bool pair_plan(const DecodeParams &p, const kitty_decode_args &a)
         return false;
     const int64_t pages = a.plan_pages > 0 && a.plan_pages < a.max_pages ? a.plan_pages : a.max_pages;
     const int64_t many = std::min<int64_t>(kPairUnitsMax, 5 * pairs / 16);
-    return pages + p.fp16_units <= std::max<int64_t>(a.plan_pages > 0 ? kPairStepUnits : kPairUnits, many);
+    return pages + p.fp16_units <= std::max<int64_t>(pair_units(p, a.plan_pages > 0), many);
 }
 
 static void sub_group(DecodeParams &p, const kitty_decode_args &a, int s);
