@@ -271,10 +271,14 @@ int kitty_paged_decode(const kitty_decode_args *args, kitty_stream_t stream);
  * kitty_paged_decode only), fp16,
  * 16-byte aligned buffers, unique boost
  * ranks) or KITTY_DECODE_PATH_GENERIC (everything else: the shape-generic
- * kernel, about 15x slower at the production shape, and, where only the
+ * kernel, 4 to 15 times slower at the production shape, and, where only the
  * element type keeps a call from the production kernel (q, sinks, tails and
- * metadata all bf16), its bf16 instance, which carries probabilities and
- * scores with the generic kernel's fp32 accuracy).  Mirrors the
+ * metadata all bf16), its bf16 instance.  That instance runs exactly where
+ * the same arguments with F16 types report MFMA, unless the workspace holds
+ * only the generic kernel's partials.  It forms q s_k in two fp16
+ * terms (all 16 bits of the product) and the probabilities in 23 bits where
+ * the generic kernel has fp32's 24; the error this adds stays below 1e-5 of the
+ * output, a twentieth of its fp16 rounding).  Mirrors the
  * dispatch decision of paged_attention (kitty/kernels/attention.py:320-341),
  * so callers can see when a profile with repeated ranks or a misaligned
  * buffer sends decode to the slower kernel. */

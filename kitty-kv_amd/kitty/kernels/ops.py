@@ -280,12 +280,12 @@ class DecodePlan:
     tail_k/v (B, Hkv, T, D) fp16 + tail_len (B,) int32; out (B, Hq, D) fp16.
     With a bfloat16 config, q, the sinks and the tails are bfloat16 and so
     are the metadata pools; out stays fp16 (the reference returns fp16,
-    kernels/attention.py:189).  ``kernel`` is "mfma" where the float16 MFMA
-    split kernel runs and "generic" for everything else: the shape-generic
-    kernel and, at the production shape with bfloat16 throughout, the bfloat16
-    instance of the MFMA kernel, which keeps the generic kernel's fp32
-    accuracy.  A production-shape plan that is not "mfma" (repeated boost
-    ranks, bf16 or misaligned buffers) warns once per process.
+    kernels/attention.py:189).  ``split_kernel`` names what runs: "mfma" (the
+    float16 MFMA kernel), "mfma_bf16" (its bfloat16 instance) or "generic" (the
+    shape-generic kernel).  ``kernel`` is the first against the rest, "mfma" or
+    "generic".  A production-shape plan that is not "mfma" warns, once per
+    process and reason (bfloat16 buffers, repeated boost ranks, mixed types,
+    misaligned buffers).
 
     Independent value stream (the KIVI split of the pipeline's FP16 value
     window): num_pages_v (B,) int32 value pages and tail_len_v (B,) int32
@@ -360,11 +360,16 @@ class DecodePlan:
         a.sm_scale = float(1.0 / math.sqrt(D) if sm_scale is None else sm_scale)
         a.meta_dtype, a.act_dtype = meta_dtype, act_dtype
         self._L = _hip.load()
-        path = ctypes.c_int32(0)
-        _hip.check(self._L.kitty_decode_path(ctypes.byref(a), ctypes.byref(path)))
-        self.kernel = "mfma" if path.value == _hip.KITTY_DECODE_PATH_MFMA else "generic"
-        if self.kernel == "generic" and D == 128 and G4 * 4 == 128 and Hq // Hkv <= 16:
-            _warn_generic(boost_unique, act_dtype, meta_dtype)
+        self.kernel = self.split_kernel = "mfma" if self._mfma(a) else "generic"
+        if act_dtype == meta_dtype == _hip.KITTY_DTYPE_BF16:
+            # the bfloat16 instance runs where float16 would run the MFMA kernel
+            as16 = _hip.DecodeArgs()
+            ctypes.memmove(ctypes.byref(as16), ctypes.byref(a), ctypes.sizeof(a))
+            as16.act_dtype = as16.meta_dtype = _hip.KITTY_DTYPE_F16
+            if self._mfma(as16):
+                self.split_kernel = "mfma_bf16"
+        if self.split_kernel != "mfma" and D == 128 and G4 * 4 == 128 and Hq // Hkv <= 16:
+            _warn_not_mfma(self.split_kernel, boost_unique, act_dtype != meta_dtype)
         need = ctypes.c_size_t(0)
         _hip.check(self._L.kitty_decode_workspace_size(ctypes.byref(a), ctypes.byref(need)))
         if workspace is None or workspace.numel() * workspace.element_size() < need.value:
@@ -379,6 +384,11 @@ class DecodePlan:
         self._keep = (q, block_table, num_pages, key_baseline, key_boost, key_meta, value_pool, value_meta,
                       boost_idx, sink_k, sink_v, sink_len, tail_k, tail_v, tail_len, workspace, num_pages_v,
                       tail_len_v)
+
+    def _mfma(self, args: _hip.DecodeArgs) -> bool:
+        path = ctypes.c_int32(0)
+        _hip.check(self._L.kitty_decode_path(ctypes.byref(args), ctypes.byref(path)))
+        return path.value == _hip.KITTY_DECODE_PATH_MFMA
 
     def run(self) -> torch.Tensor:
         _hip.check(self._L.kitty_paged_decode(ctypes.byref(self.args), _hip.stream_ptr(self.device)))
@@ -427,27 +437,28 @@ class DecodePlan:
         return self.out
 
 
-_warned_generic = False
+_warned_generic = ()      # reasons warned about
 
 
-def _warn_generic(boost_unique: bool, act_dtype: int, meta_dtype: int) -> None:
+def _warn_not_mfma(kernel: str, boost_unique: bool, mixed: bool) -> None:
     global _warned_generic
-    if _warned_generic:
-        return
-    _warned_generic = True
-    if not boost_unique:
+    if kernel == "mfma_bf16":
+        why = "the buffers are bfloat16"
+    elif not boost_unique:
         why = "a boost_idx row repeats a rank below d_boost"
-    elif act_dtype == _hip.KITTY_DTYPE_BF16 and meta_dtype == _hip.KITTY_DTYPE_BF16:
-        warnings.warn("kitty paged decode runs outside the float16 MFMA path because the buffers are bfloat16: the "
-                      "bfloat16 instance of the MFMA kernel where buffers and pools are 16-byte aligned, else the "
-                      "shape-generic kernel", RuntimeWarning, stacklevel=3)
-        return
-    elif act_dtype == _hip.KITTY_DTYPE_BF16 or meta_dtype == _hip.KITTY_DTYPE_BF16:
+    elif mixed:
         why = "only some of the buffers are bfloat16"
     else:
-        why = "a pool or FP16 buffer is not 16-byte aligned"
-    warnings.warn(f"kitty paged decode runs the shape-generic kernel because {why}; at this shape it is about "
-                  "15x slower than the MFMA kernel", RuntimeWarning, stacklevel=3)
+        why = "a pool or 16-bit buffer is not 16-byte aligned"
+    if why in (_warned_generic or ()):
+        return
+    _warned_generic = (_warned_generic or ()) + (why,)
+    if kernel == "mfma_bf16":
+        warnings.warn(f"kitty paged decode runs the bfloat16 instance of the MFMA kernel because {why}",
+                      RuntimeWarning, stacklevel=3)
+    else:
+        warnings.warn(f"kitty paged decode runs the shape-generic kernel because {why}; at this shape it is 4 to "
+                      "15 times slower than the MFMA kernel", RuntimeWarning, stacklevel=3)
 
 
 def decode_plan(*args, **kwargs):

@@ -178,3 +178,26 @@ def test_bf16_small_workspace_runs_the_generic_kernel(dev):
     plan.args.workspace_bytes = 1 << 10
     with pytest.raises(ValueError, match="workspace too small"):
         plan.run()
+
+
+@pytest.mark.gpu
+def test_bf16_plans_name_the_kernel_that_runs(dev):
+    """split_kernel tells the bfloat16 instance from the shape-generic kernel, and
+    the notice about the one does not swallow the warning about the other."""
+    import kitty.kernels.ops as ops
+    args, kw = _case(dev, 31, 8, 2, 16, [2], None, [3], [32])
+    ops._warned_generic = ()
+    with pytest.warns(RuntimeWarning, match="bfloat16 instance"):
+        plan = ops.DecodePlan(*args, **kw, boost_unique=True)
+    assert (plan.kernel, plan.split_kernel) == ("generic", "mfma_bf16")
+    off = list(args)
+    off[9] = torch.empty(args[9].numel() + 1, dtype=args[9].dtype, device=dev)[1:].view(args[9].shape)   # sink_k
+    with pytest.warns(RuntimeWarning, match="shape-generic kernel because .* aligned"):
+        plan = ops.DecodePlan(*off, **kw, boost_unique=True)
+    assert (plan.kernel, plan.split_kernel) == ("generic", "generic")
+    with pytest.warns(RuntimeWarning, match="repeats a rank"):
+        assert ops.DecodePlan(*args, **kw, boost_unique=False).split_kernel == "generic"
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")          # each once
+        ops.DecodePlan(*args, **kw, boost_unique=True)
+        ops.DecodePlan(*off, **kw, boost_unique=True)
