@@ -58,7 +58,7 @@ class KittyPagedAttention(nn.Module):
         self.scale = 1.0 / math.sqrt(config.head_dim)
         self._boost_unique = boost_rows_unique(pipeline.boost_idx_uint8[layer_id], config.d_boost)
         self._plans: dict = {}   # tuple(slots) -> DecodePlan over the pipeline's device state
-        self._steps: dict = {}   # tuple(sequence ids) -> (slot epoch, key of its plan in _plans) of its last step
+        self._steps: dict = {}   # tuple(sequence ids) -> (slot epoch, its plan in _plans) of its last step
 
     def _seq_ids(self, B: int, seq_id: Union[int, Sequence[int]]) -> List[int]:
         if isinstance(seq_id, int):
@@ -91,8 +91,9 @@ class KittyPagedAttention(nn.Module):
                           max_pages=x["max_pages"], sm_scale=self.scale, boost_unique=self._boost_unique,
                           num_pages_v=x["num_pages_v"], tail_len_v=x["tail_len_v"])
         if x["contiguous"]:      # views of the pipeline's state: valid for every later step
-            if len(self._plans) >= 16:
+            if len(self._plans) >= 16:      # bounds the workspaces: a step keeps no plan that is not here
                 self._plans.clear()
+                self._steps.clear()
             self._plans[key] = plan
         return plan
 
@@ -100,27 +101,25 @@ class KittyPagedAttention(nn.Module):
         pipe = self.pipeline
         ids = tuple(seq_ids)
         hit = self._steps.get(ids)
-        # _plans alone owns the plans and their workspaces, and bounds them
-        plan = self._plans.get(hit[1]) if hit is not None and hit[0] == pipe._slot_epoch else None
-        if plan is not None and q.dtype == pipe.buffer_dtype and q.device == pipe.device and q.is_contiguous():
+        if (hit is not None and hit[0] == pipe._slot_epoch and q.dtype == pipe.buffer_dtype and q.device == pipe.device
+                and q.is_contiguous()):
             # the batch's plan with this q and the output in q's dtype; append
             # and decode go out in one call unless this token spills
             out = torch.empty_like(q)
-            args = plan.step_args(q, out)
+            args = hit[1].step_args(q, out)
             if not pipe._push(self.layer_id, k[:, :, 0], v[:, :, 0], ids, args):
                 args.plan_pages = pipe._longest(self.layer_id, pipe._slots(ids))
-                plan.run_args(args)
+                hit[1].run_args(args)
             return out
         pipe.push_tokens(self.layer_id, k[:, :, 0], v[:, :, 0], seq_ids)
         qd = q[:, :, 0].to(pipe.buffer_dtype).contiguous()
         plan = self._plan(qd, seq_ids)
         if isinstance(plan, DecodePlan):
             plan.args.plan_pages = pipe._longest(self.layer_id, pipe._slots(ids))   # as the steps in one call
-            key = tuple(pipe.slot(s) for s in seq_ids)
-            if key in self._plans:
+            if tuple(pipe.slot(s) for s in seq_ids) in self._plans:
                 if len(self._steps) >= 64:
                     self._steps.clear()
-                self._steps[ids] = (pipe._slot_epoch, key)
+                self._steps[ids] = (pipe._slot_epoch, plan)
         out = torch.empty(qd.shape, dtype=torch.float16, device=qd.device)
         return plan.run_with(qd, out).unsqueeze(2).to(q.dtype)
 
