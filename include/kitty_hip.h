@@ -372,8 +372,9 @@ int kitty_decode_step(const kitty_append_args *append, const kitty_decode_args *
  * KITTY_E_UNSUPPORTED.  Scores that are NaN or +infinity give NaN rows, as
  * the softmax does; a NaN or infinite value reaches the rows that weigh it
  * as the product with their weights does, and may reach rows i < j of its
- * 64-token tile as NaN (weight 0 times it).  bf16 values are to stay below
- * 2^100 (the products are summed times up to 2^15). */
+ * 64-token tile as NaN (weight 0 times it).  The sum of a channel's |value|s
+ * over the prompt is to stay below 2^120 (weights up to 2^8 before they are
+ * normalised). */
 typedef struct {
     const uint16_t *q, *k, *v; /* (B, Hq, T, D), (B, Hkv, T, D) twice */
     uint16_t *out;             /* (B, Hq, T, D) */

@@ -21,8 +21,9 @@
 //
 // Probabilities keep fp32 accuracy: P enters PV as two 16-bit terms (fp16: the
 // rounded-to-zero value and its remainder, 21 bits; bf16: 16 bits), each with
-// its own MFMA, scaled by 2^7 (up to 2^15 while the running maximum lags) so
-// that small probabilities stay clear of fp16's subnormals.  The running
+// its own MFMA, in fp16 scaled by 2^7 (up to 2^15 while the running maximum lags)
+// so that small probabilities stay clear of its subnormals; bf16 has fp32's
+// exponents, and unscaled sums leave its values their range.  The running
 // maximum is raised only when a tile passes it by 2^8, so most tiles skip
 // the rescale of the 64 accumulator registers.
 //
@@ -165,7 +166,7 @@ __device__ __forceinline__ void tile_step(WaveQ &W, const unsigned char *kst, co
             for (int i = 0; i < 16; ++i)
                 W.O[dt][i] *= alpha;
     }
-    const float sub = W.m - 7.0f;
+    const float sub = BF16 ? W.m : W.m - 7.0f;
     unsigned hi[2][8], lo[2][8];
     float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll

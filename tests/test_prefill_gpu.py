@@ -158,3 +158,15 @@ def test_prefill_long_prompt_is_repeatable(dev):
         s = (k[0, h // 4, :i + 1].double() @ q[0, h, i].double()) / math.sqrt(128)
         ref = torch.softmax(s, 0) @ v[0, h // 4, :i + 1].double()
         assert ((first[0, h, i].double() - ref).abs() <= 2.0 ** -11 * ref.abs() + 1e-4).all()
+
+
+@pytest.mark.gpu
+def test_prefill_large_bf16_values(dev):
+    """bf16 values near the end of the range, as a float32 product takes them."""
+    from kitty.kernels.ops import prefill_attention
+    gen = torch.Generator().manual_seed(12)
+    q, k, v = (torch.randn(1, 1, 96, 128, generator=gen) * s for s in (0.1, 1.0, 2.0 ** 118))
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    out = prefill_attention(q.to(dev), k.to(dev), v.to(dev), 1.0 / math.sqrt(128)).cpu().double()
+    ref = _ref(q, k, v)
+    assert ((out - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4 * 2.0 ** 118).all()
