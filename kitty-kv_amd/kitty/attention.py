@@ -125,7 +125,8 @@ class KittyPagedAttention(nn.Module):
 
     def _prefill(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, seq_ids: List[int]) -> torch.Tensor:
         self.pipeline.push_chunk(self.layer_id, k, v, seq_ids)
-        if prefill_supported(q, k, v):
+        # the kernel would take any k that divides q's heads; other counts go where they raise or broadcast
+        if k.shape[1] * self.q_per_kv == q.shape[1] and prefill_supported(q, k, v):
             return prefill_attention(q, k, v, self.scale)
         k_exp = k.float().repeat_interleave(self.q_per_kv, dim=1)
         v_exp = v.float().repeat_interleave(self.q_per_kv, dim=1)

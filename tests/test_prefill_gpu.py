@@ -170,3 +170,14 @@ def test_prefill_large_bf16_values(dev):
     out = prefill_attention(q.to(dev), k.to(dev), v.to(dev), 1.0 / math.sqrt(128)).cpu().double()
     ref = _ref(q, k, v)
     assert ((out - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4 * 2.0 ** 118).all()
+
+
+@pytest.mark.gpu
+def test_module_prompt_of_other_heads_is_refused(dev):
+    from kitty import KittyAttentionFactory, KittyConfig
+    cfg = KittyConfig(num_layers=1, num_kv_heads=2, head_dim=128, max_seq_len=512, device="cuda:0")
+    bi = torch.full((1, 2, 128), cfg.sentinel, dtype=torch.uint8)
+    _, _, layers = KittyAttentionFactory.from_config(cfg, bi, 8)
+    x = lambda h: torch.randn(1, h, 20, 128, device=dev).half()
+    with pytest.raises(RuntimeError, match="must match"):
+        layers[0](x(8), x(1), x(1))
