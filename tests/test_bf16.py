@@ -169,8 +169,9 @@ def _close(got, ref, what=""):
 @pytest.mark.gpu
 def test_bf16_batched_decode_matches_oracle(dev):
     """Batched decode at the production shape with bf16 q, sinks, tails and
-    metadata pools (quantised on the device from bf16 K/V): the generic
-    kernel runs (plan.kernel, with one warning) and matches the oracle."""
+    metadata pools (quantised on the device from bf16 K/V): plan.kernel reads
+    "generic" (with one warning; the bf16 matrix-core instance runs) and the
+    output matches the oracle."""
     from kitty.kernels.ops import DecodePlan, quantize_into_pools
     gen = torch.Generator().manual_seed(21)
     B, Hq, H, D, G, Dk, S = 3, 16, 4, 128, 128, 16, 32
