@@ -365,7 +365,8 @@ int kitty_decode_step(const kitty_append_args *append, const kitty_decode_args *
  * KittyPagedAttention.forward (kitty/attention.py:179-191; ABI version 7):
  * out[b, h, i] = softmax over j <= i of (q[b, h, i] . k[b, kh, j] * sm_scale)
  * times v[b, kh, j], kh = h / (num_q_heads / num_kv_heads), with fp32 scores,
- * softmax and sums, converted to the inputs' type.  head_dim 128; q, k and v
+ * softmax and sums (weights in 21 bits for fp16, 16 for bf16), converted to the
+ * inputs' type.  head_dim 128; q, k and v
  * 16-byte aligned with strides that are multiples of 8 elements, out 8-byte
  * aligned with strides that are multiples of 4; token strides of k and v
  * non-negative with a head's rows inside 2 GiB; other layouts return

@@ -20,9 +20,10 @@ rows copied, every complete page quantised straight from the chunk in one
 launch per sequence; the same state as pushing the tokens one at a time,
 which is what the reference does, ``:169-177``), and the output is causal
 attention over the chunk, as the reference computes it (``:179-191``), with
-scores, softmax and sums in float32: fp16 and bf16 prompts at head_dim 128
+scores, softmax and sums in float32 (weights in two 16-bit terms): fp16 and bf16 prompts at head_dim 128
 run ``kitty_prefill_attention``, everything else (other head_dims, float32,
-inputs that need gradients) torch's scaled_dot_product_attention.
+inputs that need gradients, calls that are traced or transformed) torch's
+scaled_dot_product_attention.
 
 Pools and buffers on the CPU (``KittyConfig.device = "cpu"``, the reference's
 config-1 plumbing case) run the same steps with the torch code of
